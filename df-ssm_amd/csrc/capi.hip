@@ -79,7 +79,7 @@ WsLayout ws_layout(const dfssm_dims* d) {
 // residual stream of every row, the projection rows, g, the sum(g^2) slots and the prologue
 // outputs (q, scale, LoRA intermediate).
 struct PfLayout {
-  size_t x, proj, g, slots, q, xs, h, w8, total;
+  size_t x, proj, g, bc, dec, q, xs, h, w8, total;
 };
 // Prefill chunks of at least this many rows run the projections on the wide GEMM (weights
 // expanded to int8 in the prefill workspace), smaller ones on gemm_kernel.
@@ -92,7 +92,8 @@ PfLayout pf_layout(const Derived& r, int rows) {
   w.x = off;     off = align_up(off + (size_t)rows * r.D * 2);
   w.proj = off;  off = align_up(off + (size_t)rows * r.IPO * 2);
   w.g = off;     off = align_up(off + (size_t)rows * r.DI * 2);
-  w.slots = off; off = align_up(off + (size_t)rows * r.n_slots * 8);
+  w.bc = off;    off = align_up(off + (size_t)rows * 2 * r.N * 2);
+  w.dec = off;   off = align_up(off + (size_t)rows * r.H * 8);
   w.q = off;     off = align_up(off + (size_t)(rows + 15) / 16 * 16 * kq);  // rows padded to 16 (tiled)
   w.xs = off;    off = align_up(off + (size_t)rows * 4);
   w.h = off;     off = align_up(off + (size_t)rows * 16 * 4);
@@ -698,7 +699,8 @@ static int prefill_chunk(const dfssm_model* model, const int64_t* tokens, int n_
   uint16_t* xr = (uint16_t*)(pw + w.x);
   uint16_t* proj = (uint16_t*)(pw + w.proj);
   uint16_t* g = (uint16_t*)(pw + w.g);
-  double* slots = (double*)(pw + w.slots);
+  uint16_t* bc = (uint16_t*)(pw + w.bc);
+  float2* dec = (float2*)(pw + w.dec);
   EmbedArgs e{tokens, (const uint8_t*)model->emb, model->emb_scale, model->dims.emb_code == 0 ? 1 : 0, xr,
               (int*)((char*)workspace + ws_layout(&model->dims).err), r.V, r.D, n_tokens, t0, tc};
   hipError_t st = launch_embed(e, R, s);
@@ -713,8 +715,6 @@ static int prefill_chunk(const dfssm_model* model, const int64_t* tokens, int n_
       p.act = in ? xr : g;
       p.ld_act = in ? r.D : r.DI;
       p.norm_w = in ? Lw.ln_w : Lw.norm_w;
-      p.sumsq_slots = in ? nullptr : slots;
-      p.n_slots = in ? 0 : r.n_slots;
       p.lB = in ? Lw.in_lB : Lw.out_lB;
       p.lBs = in ? Lw.in_lB_s : Lw.out_lB_s;
       p.q_out = (int8_t*)(pw + w.q);
@@ -723,7 +723,7 @@ static int prefill_chunk(const dfssm_model* model, const int64_t* tokens, int n_
       p.h_out = (float*)(pw + w.h);
       p.K = in ? r.D : r.DI;
       p.q_tiled = R >= kWideGemmRows;  // the wide GEMM reads q tiled
-      st = launch_prep(p, R, in ? DFSSM_MODE_IN : DFSSM_MODE_OUT, s);
+      st = launch_prep(p, R, DFSSM_MODE_IN, s);  // (sum(g^2) from the row itself)
       if (st != hipSuccess) return hip_status(st);
       GemmArgs a{};
       a.q = (const int8_t*)(pw + w.q); a.ld_q = kq; a.M = R;
@@ -742,17 +742,20 @@ static int prefill_chunk(const dfssm_model* model, const int64_t* tokens, int n_
                               : launch_gemm(a, in ? DFSSM_MODE_IN : DFSSM_MODE_OUT, s);
       if (st != hipSuccess) return hip_status(st);
       if (!in) break;
-      ConvSeqArgs c{conv, proj + r.DI, r.IPO, Lw.conv_w, Lw.conv_b, r.C, tc};
-      st = launch_conv_seq(c, r.B, s);
+      ConvTokArgs c{};
+      c.state = conv;
+      c.xbc = proj + r.DI; c.dt = proj + r.DI + r.C; c.ld = r.IPO;
+      c.w = Lw.conv_w; c.b = Lw.conv_b; c.dt_bias = Lw.dt_bias; c.A_log = Lw.A_log;
+      c.x_out = g; c.bc_out = bc; c.dec_out = dec;
+      c.C = r.C; c.DI = r.DI; c.H = r.H; c.T = tc;
+      st = launch_conv_tokens(c, r.B, s);
       if (st != hipSuccess) return hip_status(st);
       ScanArgs sc{};
       sc.h = h;
-      sc.xbc = proj + r.DI; sc.ld_xbc = r.IPO;
-      sc.dt = proj + r.DI + r.C; sc.ld_dt = r.IPO;
+      sc.bc = bc; sc.dec = dec;
       sc.z = proj; sc.ld_z = r.IPO;
-      sc.dt_bias = Lw.dt_bias; sc.A_log = Lw.A_log; sc.D = Lw.D;
-      sc.y_out = g; sc.ld_y = r.DI;
-      sc.sumsq_slots = slots; sc.n_slots = r.n_slots;
+      sc.D = Lw.D;
+      sc.xg = g;
       sc.H = r.H; sc.P = r.P; sc.N = r.N; sc.T = tc;
       st = launch_ssm_scan(sc, r.B, s);
       if (st != hipSuccess) return hip_status(st);

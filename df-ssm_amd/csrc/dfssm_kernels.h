@@ -189,35 +189,35 @@ struct ConvArgs {
   int ld, C;
 };
 
-// Prompt prefill (prefill.hip): conv over the tokens of each sequence, rows (b, t) at b * T + t.
-struct ConvSeqArgs {
+// Prompt prefill (prefill.hip): conv + SiLU over T tokens of every sequence, and the decay factors of
+// the scan; rows (b, t) at b * T + t.
+struct ConvTokArgs {
   uint16_t* state;           // (batch, C, 3) fp16, advanced by T tokens
-  uint16_t* x;               // rows (batch * T, ld): raw xBC in, conv'd + SiLU out (in place)
+  const uint16_t* xbc;       // raw x | B | C rows (stride ld), not written
+  const uint16_t* dt;        // raw dt rows (stride ld)
   int ld;
   const uint16_t* w;         // (C, 4)
   const uint16_t* b;         // (C)
-  int C, T;
+  const float* dt_bias;      // (H)
+  const float* A_log;        // (H)
+  uint16_t* x_out;           // (batch * T, DI) conv'd x
+  uint16_t* bc_out;          // (batch * T, 2 N) conv'd B | C
+  float2* dec_out;           // (batch * T, H) {softplus dt, exp(dt A)}
+  int C, DI, H, T;
+  int tc;                    // tokens per workgroup (set by the launch)
 };
 
-// Prompt prefill: SSM + gate over T tokens per sequence (rows (b, t) at b * T + t), state in
-// registers; the fields mean what they mean in SsmArgs, with z and the slots required.
+// Prompt prefill: SSM + gate over T tokens per sequence (rows (b, t) at b * T + t), the state in
+// registers.
 struct ScanArgs {
   float* h;                  // (batch, H, P, N) fp32 state, advanced by T tokens
-  const uint16_t* xbc;       // rows x | B | C (after the conv)
-  int ld_xbc;
-  const uint16_t* dt;        // raw dt rows
-  int ld_dt;
+  const uint16_t* bc;        // (batch * T, 2 N) B | C (after the conv)
+  const float2* dec;         // (batch * T, H) {softplus dt, exp(dt A)}
   const uint16_t* z;         // gate input rows
   int ld_z;
-  const float* dt_bias;
-  const float* A_log;
-  const float* D;
-  uint16_t* y_out;           // (batch * T, ld_y) gated g
-  int ld_y;
-  double* sumsq_slots;       // (batch * T, n_slots) per-block sum(g^2)
-  int n_slots;
+  const float* D;            // (H)
+  uint16_t* xg;              // (batch * T, H P): x (after the conv) in, gated g out, in place
   int H, P, N, T;
-  int pb0;                   // set by the kernel
 };
 
 // Sampling head (sample.hip): one workgroup per sequence.
@@ -345,7 +345,7 @@ struct StateDfArgs {
   int kk, sd_bits;          // sd_bits >= 32: the error is kept unquantized
 };
 hipError_t launch_state_df(const StateDfArgs& a, hipStream_t s);
-hipError_t launch_conv_seq(const ConvSeqArgs& a, int batch, hipStream_t s);
+hipError_t launch_conv_tokens(const ConvTokArgs& a, int batch, hipStream_t s);
 hipError_t launch_ssm_scan(const ScanArgs& a, int batch, hipStream_t s);
 hipError_t launch_last_rows(const uint16_t* src, uint16_t* dst, int batch, int T, int D, hipStream_t s);
 hipError_t launch_tile_emb(const uint8_t* src, uint8_t* dst, int V, int row_bytes, hipStream_t s);

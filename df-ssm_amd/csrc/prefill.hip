@@ -1,286 +1,416 @@
 // Prompt prefill, layer-major (gfx950): the n prompt tokens of every sequence go through one
 // layer together, then the next layer. The projections and their prologues are row-independent,
-// so the decode kernels run them on all batch x n rows at once (prep_kernel, gemm_kernel); only
-// the two recurrences walk the tokens in order, here:
+// so they run on all batch x n rows at once; only the two recurrences walk the tokens, here:
 //
-//   conv_seq_kernel  one thread per (sequence, conv channel): the fp16 shift register stays in
-//                    registers while the thread walks the tokens; out = s0 w0 + s1 w1 + s2 w2 +
-//                    x w3 + b (left to right, fp32), x <- fp16(out sigmoid(out)), in place on the
-//                    projection rows, whose raw values the in_proj GEMM wrote (no conv there).
-//   ssm_scan_kernel  one workgroup per (sequence, head, up to 4 blocks of 16 state rows): the fp32
-//                    state of the rows stays in registers for all n tokens (read and written
-//                    once per layer instead of once per token). Per token the arithmetic, the
-//                    thread -> state-element map and every reduction tree are those of
-//                    ssm_kernel<true>, so state, g and the per-block sum(g^2) slots are bit-for-bit
-//                    what n decode steps produce. The tokens' operands (B | C, x, z, dt) are staged
-//                    in LDS kTT tokens at a time, double-buffered, with softplus dt, exp(dt A),
-//                    the gate factor z sigma(z), B widened to fp32 and C to fp64 computed once per
-//                    token (per row) while staging.
+//   conv_tokens_kernel  conv + SiLU of every (token, channel) from the raw projection rows:
+//                    out = s0 w0 + s1 w1 + s2 w2 + x w3 + b (left to right, fp32), fp16(out sigmoid(out)),
+//                    and the head's decay factors softplus dt, exp(dt A). x goes to the rows the scan
+//                    overwrites with g, B | C to rows of their own.
+//   ssm_scan_kernel  the SSM recurrence and the gate, one workgroup per (sequence, head, 16-row
+//                    blocks): the fp32 state stays in registers for all n tokens (read and written
+//                    once per layer instead of once per token).
 //
-// Together with the row-wise kernels this makes the prefill equal, bit for bit, to n calls of the
-// decode step (Mamba-2 recurrence of df_ssm_kernels.cu:53-103 / training/
-// df_ssm_mamba2_distill_dfw.py:346-381, evaluated token by token as the reference's
-// cpu_inference_driver.py:186-204 ingests a prompt).
-#include <type_traits>
-
+// Every rounding and every sum whose order could show is the decode step's (ssm_kernel), so
+// together with the row-wise kernels the prefill equals, bit for bit, n calls of the decode step
+// (Mamba-2 recurrence of df_ssm_kernels.cu:53-103 / training/df_ssm_mamba2_distill_dfw.py:346-381,
+// evaluated token by token as the reference's cpu_inference_driver.py:186-204 ingests a prompt).
 #include "common.h"
 #include "dfssm_kernels.h"
 
 namespace dfssm {
 
-__global__ __launch_bounds__(256) void conv_seq_kernel(ConvSeqArgs a) {
-  const int ch = blockIdx.x * 256 + threadIdx.x;
-  const int b = blockIdx.y;
+// The caller's conv tensors carry no alignment beyond their 2-byte elements (the address mode of the
+// target takes a vector access at any address).
+typedef u32x4 u32x4_a2 __attribute__((aligned(2)));
+
+// ------------------------------------------------------------------------------------------
+// conv_tokens_kernel: a thread owns 8 channels and walks tc tokens (16-byte rows in and out), the
+// three raw inputs before its first token re-read from the rows (or the conv state). The tokens
+// of a sequence are independent once the raw rows are kept, so they spread over the grid: a thread
+// that walked the whole sequence with the outputs in place took 208 us for 999 tokens of one
+// sequence at the 1.3B shape (17 workgroups on the chip), this one 18 us. The first token range also writes the new
+// conv state, the last three raw inputs. The last block of the x grid computes the decay factors of
+// its tokens, one (token, head) per thread.
+// ------------------------------------------------------------------------------------------
+__global__ __launch_bounds__(256) void conv_tokens_kernel(ConvTokArgs a) {
+  const int tid = threadIdx.x, b = blockIdx.z;
+  const int t0 = (int)blockIdx.y * a.tc, t1 = t0 + a.tc < a.T ? t0 + a.tc : a.T;
+  const size_t row0 = (size_t)b * a.T;
+  if (blockIdx.x == gridDim.x - 1) {
+    for (int i = tid; i < (t1 - t0) * a.H; i += 256) {
+      const int t = t0 + i / a.H, hd = i % a.H;
+      const float dt = dev_log1pf(dev_expf(h2f(a.dt[(row0 + t) * a.ld + hd]) + a.dt_bias[hd]));
+      a.dec_out[(row0 + t) * a.H + hd] = float2{dt, dev_expf(dt * -dev_expf(a.A_log[hd]))};
+    }
+    return;
+  }
+  const int ch = 8 * ((int)blockIdx.x * 256 + tid);
   if (ch >= a.C) return;
-  uint16_t* cs = a.state + ((size_t)b * a.C + ch) * 3;
-  uint16_t s0 = cs[0], s1 = cs[1], s2 = cs[2];
-  const uint16_t* wc = a.w + (size_t)ch * 4;
-  const float w0 = h2f(wc[0]), w1 = h2f(wc[1]), w2 = h2f(wc[2]), w3 = h2f(wc[3]);
-  const float cb = h2f(a.b[ch]);
-  uint16_t* col = a.x + (size_t)b * a.T * a.ld + ch;  // token t of sequence b: col[t * ld]
-  constexpr int U = 8;
-  for (int t0 = 0; t0 < a.T; t0 += U) {
-    uint16_t raw[U];
+  const uint16_t* raw = a.xbc + row0 * a.ld + ch;
+  u32x4 wr[4];
 #pragma unroll
-    for (int u = 0; u < U; ++u) raw[u] = col[(size_t)(t0 + u < a.T ? t0 + u : a.T - 1) * a.ld];
+  for (int i = 0; i < 4; ++i) wr[i] = *(const u32x4_a2*)(a.w + (size_t)ch * 4 + 8 * i);
+  const u32x4 br = *(const u32x4_a2*)(a.b + ch);
+  uint16_t s[3][8];  // the three inputs before the current token
+  u32x4_a2* cs = (u32x4_a2*)(a.state + ((size_t)b * a.C + ch) * 3);  // 8 channels x 3 halves
+  if (t0 == 0) {
+    const u32x4 st[3] = {cs[0], cs[1], cs[2]};
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      if (t0 + u >= a.T) break;
-      const uint16_t xo = raw[u];
-      float o = h2f(s0) * w0;
-      o = o + h2f(s1) * w1;
-      o = o + h2f(s2) * w2;
-      o = o + h2f(xo) * w3;
-      o = o + cb;
-      const float sig = 1.0f / (1.0f + dev_expf(-o));
-      col[(size_t)(t0 + u) * a.ld] = f2h(o * sig);
-      s0 = s1;
-      s1 = s2;
-      s2 = xo;
+    for (int e = 0; e < 8; ++e)
+#pragma unroll
+      for (int k = 0; k < 3; ++k) s[k][e] = (uint16_t)(st[(3 * e + k) >> 3][((3 * e + k) & 7) >> 1] >> (16 * ((3 * e + k) & 1)));
+  } else {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const u32x4 v = *(const u32x4*)(raw + (size_t)(t0 - 3 + k) * a.ld);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) s[k][e] = (uint16_t)(v[e >> 1] >> (16 * (e & 1)));
     }
   }
-  cs[0] = s0;
-  cs[1] = s1;
-  cs[2] = s2;
+  if (t0 == 0) {  // the conv state after the sequence (nobody else reads or writes it)
+    uint16_t n[3][8];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const int t = a.T - 3 + k;
+      const u32x4 v = *(const u32x4*)(raw + (size_t)(t < 0 ? 0 : t) * a.ld);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const uint16_t keep = a.T + k < 3 ? s[a.T == 1 ? (k + 1 > 2 ? 2 : k + 1) : 2][e] : (uint16_t)0;
+        n[k][e] = t < 0 ? keep : (uint16_t)(v[e >> 1] >> (16 * (e & 1)));
+      }
+    }
+    u32x4 o[3] = {};
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+#pragma unroll
+      for (int k = 0; k < 3; ++k) o[(3 * e + k) >> 3][((3 * e + k) & 7) >> 1] |= (uint32_t)n[k][e] << (16 * ((3 * e + k) & 1));
+#pragma unroll
+    for (int i = 0; i < 3; ++i) cs[i] = o[i];
+  }
+  const bool is_x = ch < a.DI;  // (DI is a multiple of 8)
+  uint16_t* out = is_x ? a.x_out + row0 * a.DI + ch : a.bc_out + row0 * (a.C - a.DI) + (ch - a.DI);
+  const int ld_out = is_x ? a.DI : a.C - a.DI;
+  u32x4 nx = *(const u32x4*)(raw + (size_t)t0 * a.ld);
+  for (int t = t0; t < t1; ++t) {
+    const u32x4 v = nx;
+    nx = *(const u32x4*)(raw + (size_t)(t + 1 < t1 ? t + 1 : t) * a.ld);
+    u32x4 o = {0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const uint16_t xo = (uint16_t)(v[e >> 1] >> (16 * (e & 1)));
+      const uint32_t w01 = wr[e >> 1][2 * (e & 1)], w23 = wr[e >> 1][2 * (e & 1) + 1];
+      float f = h2f(s[0][e]) * h2f((uint16_t)w01);
+      f = f + h2f(s[1][e]) * h2f((uint16_t)(w01 >> 16));
+      f = f + h2f(s[2][e]) * h2f((uint16_t)w23);
+      f = f + h2f(xo) * h2f((uint16_t)(w23 >> 16));
+      f = f + h2f((uint16_t)(br[e >> 1] >> (16 * (e & 1))));
+      const float sig = 1.0f / (1.0f + dev_expf(-f));
+      o[e >> 1] |= (uint32_t)f2h(f * sig) << (16 * (e & 1));
+      s[0][e] = s[1][e];
+      s[1][e] = s[2][e];
+      s[2][e] = xo;
+    }
+    *(u32x4*)(out + (size_t)t * ld_out) = o;
+  }
 }
 
-constexpr int kTT = 16;    // tokens staged per round
-constexpr int kPGMax = 4;  // 16-row state blocks per workgroup
-constexpr int kTG = 4;     // tokens whose reductions run together
+// ------------------------------------------------------------------------------------------
+// ssm_scan_kernel<W, RB>: RB 16-row blocks of one head per workgroup, W waves per block.
+//
+// What bounds it is VALU issue: a state element takes four instructions per token (x dt B, the fma
+// of the state, the widening of h and the fp64 fma of the readout), and everything else is kept
+// off the elements. Lane (g, r) = (lane / 16, lane % 16) of a wave holds row r of the block and
+// 32 / W of its 128 state columns; the four lane groups (and the W waves) hold the others. So
+// * B and C are the same for the 16 lanes of a group: each lane reads one pair of columns per token
+//   from LDS (widened while staging) and the multiply and the fp64 fma take the other lanes' pairs
+//   as DPP row broadcasts, at no cost;
+// * one row sum per token and lane crosses lanes, and the sums of four tokens together: the lane
+//   swaps of gfx950 exchange two tokens' values between lane groups (reduce4), after which lane
+//   group g holds token t + g's sums, so the readout, the gate and the store run once per four
+//   tokens on full waves.
+// Measured per layer, against the map this replaces (ssm_kernel's own, two rows and four columns per
+// lane, whose reductions took two thirds of the instructions and which kept a head on one CU):
+// 4796 -> 1499 us at the 2.7B shape and 64 x 256 tokens (1.07 ms if the four instructions per
+// element issued back to back), 916 -> 187 us at the 1.3B shape and 1 x 999 tokens (W = 4), 32.6 ->
+// 9.4 us at 1 x 32.
+//
+// The readout's sum is ssm_kernel's tree: quads A_j of four columns summed in order from zero (the
+// product C h is exact in fp64, so an fma rounds as its multiply-then-add), Q_i = (A_4i + A_4i+1) +
+// (A_4i+2 + A_4i+3), then ((Q0 + Q3) + (Q2 + Q1)) + ((Q4 + Q7) + (Q6 + Q5)). The columns are dealt
+// out so that the tree's levels are, from the inside: the lane, the lane groups 16 lanes apart, 32
+// lanes apart, the waves:
+//   W = 1: group g holds Q_2g and Q_(2g ^ 3);
+//   W = 2: wave w holds Q_4w .. Q_4w+3, group g Q_4w + (-g mod 4);
+//   W = 4: wave w holds Q_2w (groups 0, 1: its halves) and Q_(2w ^ 3) (groups 2, 3).
+// More waves per block cost more instructions per element (the per-token work is shared by fewer
+// columns) and a partial sum through LDS, but fill the chip when there are few blocks
+// (launch_ssm_scan).
+//
+// Rounds of TT tokens are staged in LDS, double-buffered, their operands loaded one round ahead.
+// ------------------------------------------------------------------------------------------
+constexpr int scan_tt(int W) { return W == 1 ? 8 : 4 * W; }  // tokens per round
 
+template <int W, int RB>
 struct ScanBuf {
-  float bf[kTT][128];              // B of each token, widened once here (fp16 values)
-  double cd[kTT][128];             // C of each token, widened to fp64 (fp16 values)
-  uint16_t x[kTT][16 * kPGMax];    // x of the workgroup's rows
-  float sz[kTT][16 * kPGMax];      // gate factor fp16(z sigma(z)) of the workgroup's rows
-  float dt[kTT], abar[kTT];        // softplus dt and exp(dt A) of the head
-  double gpart[kTT][4 * kPGMax];   // per-wave partial sum(g^2), reduced per block after the round
+  static constexpr int TT = scan_tt(W);
+  float bf[TT][128];       // B of each token, widened
+  double cd[TT][128];      // C of each token, widened
+  float X[TT][16 * RB];    // x dt of the workgroup's rows
+  float abar[TT];          // exp(dt A)
+  double part[W > 1 ? W : 1][W > 1 ? TT : 1][16 * RB];  // the waves' row sums
 };
 
-// Raw operands of one round, loaded into registers one round ahead.
-template <int PG>
+// Raw operands of one round, loaded into registers one round ahead. A thread's items are the
+// (token, row) pairs it finishes: W = 1: its lane's row and tokens 4 k + g; W > 1: one item per
+// thread, token tid / (16 RB), row tid % (16 RB).
+template <int W, int RB>
 struct ScanRaw {
-  static constexpr int KB = (kTT * 32 + 256 * PG - 1) / (256 * PG);
-  u32x4 bc[KB];    // 8 halves of B | C: chunk i = tid + 256 PG k, token i / 32, halves 8 (i % 32) ..
-  uint16_t x, z;   // token tid / (16 PG), row tid % (16 PG) (tid < kTT * 16 PG = blockDim)
-  uint16_t dt;     // token tid (tid < kTT)
+  static constexpr int NT = 64 * W * RB, TT = scan_tt(W);
+  static constexpr int NI = TT * 16 * RB / NT;        // items per thread
+  static constexpr int NB = TT * 32 / NT;             // 16-byte vectors of B | C per thread
+  static_assert(NI * NT == TT * 16 * RB && NB * NT == TT * 32, "whole vectors and items per thread");
+  u32x4 bc[NB];
+  uint16_t x[NI], z[NI];
+  float dt[NI];
+  float abar;  // token tid % TT
 };
 
-template <int PG>
-__device__ __forceinline__ ScanRaw<PG> scan_load(const ScanArgs& a, int b, int head, int t0) {
+template <int W, int RB>
+__device__ __forceinline__ int scan_item_token(int k) {
+  return W == 1 ? 4 * k + (((int)threadIdx.x & 63) >> 4) : (int)threadIdx.x / (16 * RB);
+}
+template <int W, int RB>
+__device__ __forceinline__ int scan_item_row() {
+  return W == 1 ? 16 * ((int)threadIdx.x >> 6) + ((int)threadIdx.x & 15) : (int)threadIdx.x % (16 * RB);
+}
+// Vector i of a round's B | C: token and 8-column block of B (below 16) or C; the order keeps a
+// wave's vectors all B or all C
+template <int TT>
+__device__ __forceinline__ void scan_bc_pos(int i, int& t, int& c) {
+  t = (i % (16 * TT)) / 16;
+  c = (i / (16 * TT)) * 16 + i % 16;
+}
+
+template <int W, int RB>
+__device__ __forceinline__ ScanRaw<W, RB> scan_load(const ScanArgs& a, int b, int head, int col0, int t0) {
+  using Raw = ScanRaw<W, RB>;
   const int tid = threadIdx.x;
-  constexpr int NT = 256 * PG, RW = 16 * PG;
-  ScanRaw<PG> r{};
-  const size_t row0 = (size_t)b * a.T;
-  // clamped token indices: rows past the end re-read the last token (never consumed)
+  Raw r;
+  // clamped token indices: tokens past the end re-read the last one (never consumed). 32-bit element
+  // offsets: at most 32768 rows of under 32768 elements.
+  auto row = [&](int t) { return (uint32_t)(b * a.T + (t < a.T ? t : a.T - 1)); };
 #pragma unroll
-  for (int k = 0; k < ScanRaw<PG>::KB; ++k) {
-    const int i = tid + NT * k;
-    const int t = t0 + i / 32;
-    const uint16_t* p = a.xbc + (row0 + (t < a.T ? t : a.T - 1)) * a.ld_xbc + a.H * a.P + 8 * (i % 32);
-    if (i < kTT * 32) r.bc[k] = *(const u32x4*)p;
+  for (int k = 0; k < Raw::NB; ++k) {
+    int t, c;
+    scan_bc_pos<Raw::TT>(tid + Raw::NT * k, t, c);
+    r.bc[k] = *(const u32x4*)(a.bc + (row(t0 + t) * 256u + 8u * c));
   }
-  if (tid < kTT * RW) {
-    const int t = t0 + tid / RW;
-    const size_t row = row0 + (t < a.T ? t : a.T - 1);
-    const int col = head * a.P + a.pb0 * 16 + tid % RW;
-    r.x = a.xbc[row * a.ld_xbc + col];
-    r.z = a.z[row * a.ld_z + col];
+  const uint32_t col = col0 + scan_item_row<W, RB>();
+#pragma unroll
+  for (int k = 0; k < Raw::NI; ++k) {
+    const uint32_t m = row(t0 + scan_item_token<W, RB>(k));
+    r.x[k] = a.xg[m * (uint32_t)(a.H * a.P) + col];
+    r.z[k] = a.z[m * (uint32_t)a.ld_z + col];
+    r.dt[k] = a.dec[m * (uint32_t)a.H + head].x;
   }
-  if (tid < kTT) {
-    const int t = t0 + tid;
-    r.dt = a.dt[(row0 + (t < a.T ? t : a.T - 1)) * a.ld_dt + head];
-  }
+  r.abar = a.dec[row(t0 + tid % Raw::TT) * (uint32_t)a.H + head].y;
   return r;
 }
 
-template <int PG>
-__device__ __forceinline__ void scan_stage(ScanBuf& S, const ScanRaw<PG>& r, float dtb, float nA) {
+template <int W, int RB>
+__device__ __forceinline__ void scan_stage(ScanBuf<W, RB>& S, const ScanRaw<W, RB>& r) {
+  using Raw = ScanRaw<W, RB>;
   const int tid = threadIdx.x;
-  constexpr int NT = 256 * PG, RW = 16 * PG;
 #pragma unroll
-  for (int k = 0; k < ScanRaw<PG>::KB; ++k) {
-    const int i = tid + NT * k;
-    if (i < kTT * 32) {
-      const int t = i / 32, c = i % 32;  // halves 8 c .. 8 c + 7 of B | C
-      const u32x4 v = r.bc[k];
-      float f[8];
+  for (int k = 0; k < Raw::NB; ++k) {
+    int t, c;
+    scan_bc_pos<Raw::TT>(tid + Raw::NT * k, t, c);
+    float f[8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) f[e] = h2f((uint16_t)(v[e >> 1] >> (16 * (e & 1))));
-      if (c < 16) {
-        *(f32x4*)&S.bf[t][8 * c] = f32x4{f[0], f[1], f[2], f[3]};
-        *(f32x4*)&S.bf[t][8 * c + 4] = f32x4{f[4], f[5], f[6], f[7]};
-      } else {
-        double* d = &S.cd[t][8 * (c - 16)];
+    for (int e = 0; e < 8; ++e) f[e] = h2f((uint16_t)(r.bc[k][e >> 1] >> (16 * (e & 1))));
+    if (c < 16) {
+      *(f32x4*)&S.bf[t][8 * c] = f32x4{f[0], f[1], f[2], f[3]};
+      *(f32x4*)&S.bf[t][8 * c + 4] = f32x4{f[4], f[5], f[6], f[7]};
+    } else {
+      double* d = &S.cd[t][8 * (c - 16)];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) d[e] = (double)f[e];
-      }
+      for (int e = 0; e < 8; ++e) d[e] = (double)f[e];
     }
   }
-  if (tid < kTT * RW) {
-    const int t = tid / RW, i = tid % RW;
-    S.x[t][i] = r.x;
-    const float z = h2f(r.z);
-    S.sz[t][i] = r16(z * r16(1.0f / (1.0f + dev_expf(-z))));
-  }
-  if (tid < kTT) {
-    const float dt = dev_log1pf(dev_expf(h2f(r.dt) + dtb));
-    S.dt[tid] = dt;
-    S.abar[tid] = dev_expf(dt * nA);
-  }
+#pragma unroll
+  for (int k = 0; k < Raw::NI; ++k) S.X[scan_item_token<W, RB>(k)][scan_item_row<W, RB>()] = h2f(r.x[k]) * r.dt[k];
+  if (tid < Raw::TT) S.abar[tid] = r.abar;
 }
 
-// v of lane l + 16 in lanes 0..15 and 32..47, and of lane l + 32 in lanes 0..31, by the gfx950
-// lane swaps (v_permlane16_swap between rows 0|1 and 2|3, v_permlane32_swap between the halves;
-// with both operands v, the second result holds the partner row's value in rows 0 and 2).
-__device__ __forceinline__ double lane_plus16(double v) {
-  const uint64_t u = __builtin_bit_cast(uint64_t, v);
-  const uint32_t lo = __builtin_amdgcn_permlane16_swap((uint32_t)u, (uint32_t)u, false, false)[1];
-  const uint32_t hi = __builtin_amdgcn_permlane16_swap((uint32_t)(u >> 32), (uint32_t)(u >> 32), false, false)[1];
-  return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
-}
-__device__ __forceinline__ double lane_plus32(double v) {
-  const uint64_t u = __builtin_bit_cast(uint64_t, v);
-  const uint32_t lo = __builtin_amdgcn_permlane32_swap((uint32_t)u, (uint32_t)u, false, false)[1];
-  const uint32_t hi = __builtin_amdgcn_permlane32_swap((uint32_t)(u >> 32), (uint32_t)(u >> 32), false, false)[1];
-  return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+// Quads 2 I and 2 I + 1 of one token: the state updates (in place) and the quads' fp64 sums. b0, b1 /
+// c0, c1: this lane's pair of columns of B / C; lanes 4 I .. 4 I + 3 of its row hold the eight columns.
+// In asm because the fp64 fma with a row broadcast has no builtin, and so that the state stays in its
+// registers. The first two instructions write none of the registers the DPP reads come from, which
+// covers the two wait states between a VALU write and a DPP read, whatever precedes the block; two
+// independent chains throughout.
+template <int I>
+__device__ __forceinline__ void scan_quads(float* h, float abar, float X, float b0, float b1, double c0, double c1,
+                                           double& s0, double& s1) {
+  float t0, t1, t2, t3;
+  double d0, d1, d2, d3;
+#define DFSSM_ROW(n) " row_newbcast:" n " row_mask:0xf bank_mask:0xf\n\t"
+  asm("v_mov_b64 %0, 0\n\t"
+      "v_mov_b64 %1, 0\n\t"
+      "v_mul_f32_dpp %10, %20, %19" DFSSM_ROW("%24")
+      "v_mul_f32_dpp %11, %20, %19" DFSSM_ROW("%26")
+      "v_mul_f32_dpp %12, %21, %19" DFSSM_ROW("%24")
+      "v_mul_f32_dpp %13, %21, %19" DFSSM_ROW("%26")
+      "v_fma_f32 %2, %18, %2, %10\n\t"
+      "v_fma_f32 %6, %18, %6, %11\n\t"
+      "v_fma_f32 %3, %18, %3, %12\n\t"
+      "v_fma_f32 %7, %18, %7, %13\n\t"
+      "v_cvt_f64_f32 %14, %2\n\t"
+      "v_cvt_f64_f32 %15, %6\n\t"
+      "v_cvt_f64_f32 %16, %3\n\t"
+      "v_cvt_f64_f32 %17, %7\n\t"
+      "v_mul_f32_dpp %10, %20, %19" DFSSM_ROW("%25")
+      "v_mul_f32_dpp %11, %20, %19" DFSSM_ROW("%27")
+      "v_fmac_f64_dpp %0, %22, %14" DFSSM_ROW("%24")
+      "v_fmac_f64_dpp %1, %22, %15" DFSSM_ROW("%26")
+      "v_mul_f32_dpp %12, %21, %19" DFSSM_ROW("%25")
+      "v_mul_f32_dpp %13, %21, %19" DFSSM_ROW("%27")
+      "v_fma_f32 %4, %18, %4, %10\n\t"
+      "v_fma_f32 %8, %18, %8, %11\n\t"
+      "v_fmac_f64_dpp %0, %23, %16" DFSSM_ROW("%24")
+      "v_fmac_f64_dpp %1, %23, %17" DFSSM_ROW("%26")
+      "v_fma_f32 %5, %18, %5, %12\n\t"
+      "v_fma_f32 %9, %18, %9, %13\n\t"
+      "v_cvt_f64_f32 %14, %4\n\t"
+      "v_cvt_f64_f32 %15, %8\n\t"
+      "v_cvt_f64_f32 %16, %5\n\t"
+      "v_cvt_f64_f32 %17, %9\n\t"
+      "v_fmac_f64_dpp %0, %22, %14" DFSSM_ROW("%25")
+      "v_fmac_f64_dpp %1, %22, %15" DFSSM_ROW("%27")
+      "v_fmac_f64_dpp %0, %23, %16" DFSSM_ROW("%25")
+      "v_fmac_f64_dpp %1, %23, %17" DFSSM_ROW("%27")
+      : "=&v"(s0), "=&v"(s1), "+v"(h[0]), "+v"(h[1]), "+v"(h[2]), "+v"(h[3]), "+v"(h[4]), "+v"(h[5]), "+v"(h[6]),
+        "+v"(h[7]), "=&v"(t0), "=&v"(t1), "=&v"(t2), "=&v"(t3), "=&v"(d0), "=&v"(d1), "=&v"(d2), "=&v"(d3)
+      : "v"(abar), "v"(X), "v"(b0), "v"(b1), "v"(c0), "v"(c1), "n"(4 * I), "n"(4 * I + 1), "n"(4 * I + 2), "n"(4 * I + 3));
+#undef DFSSM_ROW
 }
 
-template <int PG>
-__global__ __launch_bounds__(256 * PG) void ssm_scan_kernel(ScanArgs a) {
-  __shared__ ScanBuf buf[2];
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int grp = tid >> 8;            // 16-row block of this thread within the workgroup
-  const int gt = tid & 255;            // thread within its block: the ssm_kernel map
+// The lane swaps on fp64 values: a's odd 16-lane rows change places with b's even ones; a's upper
+// 32 lanes with b's lower ones.
+__device__ __forceinline__ void swap16_f64(double& a, double& b) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, a), v = __builtin_bit_cast(uint64_t, b);
+  const auto lo = __builtin_amdgcn_permlane16_swap((uint32_t)u, (uint32_t)v, false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap((uint32_t)(u >> 32), (uint32_t)(v >> 32), false, false);
+  a = __builtin_bit_cast(double, ((uint64_t)hi[0] << 32) | lo[0]);
+  b = __builtin_bit_cast(double, ((uint64_t)hi[1] << 32) | lo[1]);
+}
+__device__ __forceinline__ void swap32_f64(double& a, double& b) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, a), v = __builtin_bit_cast(uint64_t, b);
+  const auto lo = __builtin_amdgcn_permlane32_swap((uint32_t)u, (uint32_t)v, false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap((uint32_t)(u >> 32), (uint32_t)(v >> 32), false, false);
+  a = __builtin_bit_cast(double, ((uint64_t)hi[0] << 32) | lo[0]);
+  b = __builtin_bit_cast(double, ((uint64_t)hi[1] << 32) | lo[1]);
+}
+// Lane group g's result: (v_g of group 0 + of group 1) + (of group 2 + of group 3), row by row.
+__device__ __forceinline__ double reduce4(double v0, double v1, double v2, double v3) {
+  swap16_f64(v0, v1);
+  swap16_f64(v2, v3);
+  double a = v0 + v1, b = v2 + v3;
+  swap32_f64(a, b);
+  return a + b;
+}
+
+template <int W, int RB>
+__global__ __launch_bounds__(64 * W * RB, 4) void ssm_scan_kernel(ScanArgs a) {
+  using Buf = ScanBuf<W, RB>;
+  using Raw = ScanRaw<W, RB>;
+  constexpr int TT = Buf::TT, NQ = 8 / W;  // tokens per round; quads per lane
+  __shared__ Buf buf[2];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int blk = wave / W, w = wave % W;  // 16-row block within the workgroup; wave of the block
+  const int g = lane >> 4, r = lane & 15;
   const int b = blockIdx.y;
-  const int wg_per_head = a.P / (16 * PG);
-  const int head = blockIdx.x / wg_per_head;
-  const int pb = (blockIdx.x % wg_per_head) * PG + grp;  // state block of this thread
-  ScanArgs aa = a;
-  aa.pb0 = (blockIdx.x % wg_per_head) * PG;
-  const int n0 = 4 * (gt & 31);
-  const int pr = gt >> 5;              // rows pr and pr + 8 of the block
-  const int p = pb * 16 + pr;
-  const int rl = grp * 16 + pr;        // row index within the workgroup's staged x / sz
-  const float Dh = a.D[head], dtb = a.dt_bias[head];
-  const float nA = -dev_expf(a.A_log[head]);
+  const int wg_per_head = a.P / (16 * RB);
+  const int head = (int)blockIdx.x / wg_per_head;
+  const int p0 = ((int)blockIdx.x % wg_per_head) * (16 * RB);  // first row of the workgroup in the head
+  const int col0 = head * a.P + p0;
+  const int rl = 16 * blk + r;
+  const float Dh = a.D[head];
+  // this lane's columns: quads 4 q .. of Qa and Qb, and its pair of columns for the broadcasts
+  const int Qa = W == 1 ? 2 * g : W == 2 ? 4 * w + ((4 - g) & 3) : (g < 2 ? 2 * w : (2 * w) ^ 3);
+  const int Qb = W == 1 ? Qa ^ 3 : Qa;
+  const int half = W == 4 ? 8 * (g & 1) : 0;
+  const int pair = W == 1 ? (r < 8 ? 8 * Qa + r : 8 * Qb + r - 8) : W == 2 ? 8 * Qa + (r & 7) : 8 * Qa + half / 2 + (r & 3);
 
-  ScanRaw<PG> raw = scan_load<PG>(aa, b, head, 0);
-  float* hp = a.h + (((size_t)b * a.H + head) * a.P + p) * a.N + n0;
-  const f32x4 s0 = ld_nt_f4(hp);
-  const f32x4 s1 = ld_nt_f4(hp + 8 * a.N);
-  float h0[4] = {s0.x, s0.y, s0.z, s0.w}, h1[4] = {s1.x, s1.y, s1.z, s1.w};
-  scan_stage<PG>(buf[0], raw, dtb, nA);
+  Raw raw = scan_load<W, RB>(a, b, head, col0, 0);
+  float* hp = a.h + (((size_t)b * a.H + head) * a.P + p0 + rl) * a.N;
+  float h[4 * NQ];
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    const f32x4 v = ld_nt_f4(hp + 16 * (q < 4 ? Qa : Qb) + half + 4 * (q & 3));
+    h[4 * q] = v.x; h[4 * q + 1] = v.y; h[4 * q + 2] = v.z; h[4 * q + 3] = v.w;
+  }
+  scan_stage<W, RB>(buf[0], raw);
   lds_barrier();
 
-  const int rounds = (a.T + kTT - 1) / kTT;
+  const int rounds = (a.T + TT - 1) / TT;
   for (int rd = 0; rd < rounds; ++rd) {
-    const int t0 = rd * kTT;
-    ScanBuf& S = buf[rd & 1];
-    if (rd + 1 < rounds) raw = scan_load<PG>(aa, b, head, t0 + kTT);
-    const int nt = a.T - t0 < kTT ? a.T - t0 : kTT;
-    // Tokens in groups of kTG: the state updates are a chain of fmas, but a token's readout and
-    // sum(g^2) reductions feed nothing later, so a group's reductions are independent chains the
-    // compiler interleaves. Slots of a group past nt update nothing and store nothing.
-    for (int t = 0; t < nt; t += kTG) {
-      double acc0[kTG], acc1[kTG];
-      float xv0[kTG], xv1[kTG];
-      // FULL: all kTG tokens of the group exist (every group but a prompt's last), no selects
-      auto group = [&](auto full_t) {
-        constexpr bool FULL = decltype(full_t)::value;
+    const int t0 = rd * TT;
+    Buf& S = buf[rd & 1];
+    // this round's items, kept for the gate, and the next round's operands on their way (past the
+    // last round a re-read that nobody consumes: a branch would make the loads' users wait)
+    const Raw cur = raw;
+    raw = scan_load<W, RB>(a, b, head, col0, t0 + TT);
+    const int nt = a.T - t0 < TT ? a.T - t0 : TT;
+    auto finish = [&](double s, int k) {  // item k of this thread from its row's readout
+      const int t = scan_item_token<W, RB>(k);
+      const float z = h2f(cur.z[k]);
+      const float sz = r16(z * r16(1.0f / (1.0f + dev_expf(-z))));
+      const float y = r16((float)s + h2f(cur.x[k]) * Dh);
+      if (t < nt) a.xg[((size_t)b * a.T + t0 + t) * (a.H * a.P) + col0 + scan_item_row<W, RB>()] = f2h(y * sz);
+    };
 #pragma unroll
-        for (int j = 0; j < kTG; ++j) {
-          const int tt = FULL ? t + j : (t + j < nt ? t + j : t);
-          const f32x4 b4 = *(const f32x4*)&S.bf[tt][n0];
-          const float bq[4] = {b4.x, b4.y, b4.z, b4.w};
-          const double* cp = &S.cd[tt][n0];
-          const double cq[4] = {cp[0], cp[1], cp[2], cp[3]};
-          const float dt = S.dt[tt], abar = S.abar[tt];
-          xv0[j] = h2f(S.x[tt][rl]);
-          xv1[j] = h2f(S.x[tt][rl + 8]);
-          const float X0 = xv0[j] * dt, X1 = xv1[j] * dt;
-          const bool valid = FULL || t + j < nt;
-          acc0[j] = 0.0;
-          acc1[j] = 0.0;
+    for (int k = 0; k < TT / 4; ++k) {
+      if (4 * k >= nt) break;
+      double acc[4];
 #pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const float n0v = __builtin_fmaf(abar, h0[q], X0 * bq[q]);
-            const float n1v = __builtin_fmaf(abar, h1[q], X1 * bq[q]);
-            h0[q] = valid ? n0v : h0[q];
-            h1[q] = valid ? n1v : h1[q];
-            // C h is exact in fp64 (11 x 24 significant bits), so the fma rounds exactly as
-            // ssm_kernel's multiply-then-add
-            acc0[j] = __builtin_fma(cq[q], (double)h0[q], acc0[j]);
-            acc1[j] = __builtin_fma(cq[q], (double)h1[q], acc1[j]);
-          }
+      for (int j = 0; j < 4; ++j) {
+        const int t = 4 * k + j;
+        acc[j] = 0.0;
+        if (t >= nt) continue;  // uniform: past the prompt's end
+        const float2 bp = *(const float2*)&S.bf[t][2 * pair];
+        const double c0 = S.cd[t][2 * pair], c1 = S.cd[t][2 * pair + 1];
+        const float X = S.X[t][rl], abar = S.abar[t];
+        double A[8 / W];
+        scan_quads<0>(h, abar, X, bp.x, bp.y, c0, c1, A[0], A[1]);
+        double q = A[0] + A[1];
+        if constexpr (NQ > 2) {
+          scan_quads<1>(h + 8, abar, X, bp.x, bp.y, c0, c1, A[2], A[3]);
+          q = q + (A[2] + A[3]);
         }
-      };
-      if (t + kTG <= nt) group(std::true_type{});
-      else group(std::false_type{});
-#pragma unroll
-      for (int j = 0; j < kTG; ++j) {
-        acc0[j] = row_sum_f64(acc0[j]);
-        acc1[j] = row_sum_f64(acc1[j]);
-      }
-      double gsqd[kTG];
-#pragma unroll
-      for (int j = 0; j < kTG; ++j) {
-        // the two 16-lane row sums of each state row added as ssm_kernel's readlanes add them:
-        // (lane 0) + (lane 16) in lane 0, (lane 32) + (lane 48) in lane 32
-        const double s0 = acc0[j] + lane_plus16(acc0[j]);
-        const double s1 = acc1[j] + lane_plus16(acc1[j]);
-        gsqd[j] = 0.0;
-        if ((gt & 31) == 0 && t + j < nt) {
-          const float y0 = r16((float)s0 + xv0[j] * Dh);
-          const float y1 = r16((float)s1 + xv1[j] * Dh);
-          const float o0 = r16(y0 * S.sz[t + j][rl]);
-          const float o1 = r16(y1 * S.sz[t + j][rl + 8]);
-          gsqd[j] = (double)o0 * (double)o0 + (double)o1 * (double)o1;
-          uint16_t* yp = a.y_out + ((size_t)b * a.T + t0 + t + j) * a.ld_y + head * a.P + p;
-          yp[0] = f2h(o0);
-          yp[8] = f2h(o1);
+        if constexpr (NQ > 4) {
+          scan_quads<2>(h + 16, abar, X, bp.x, bp.y, c0, c1, A[4], A[5]);
+          scan_quads<3>(h + 24, abar, X, bp.x, bp.y, c0, c1, A[6], A[7]);
+          q = q + ((A[4] + A[5]) + (A[6] + A[7]));
         }
+        acc[j] = q;
       }
-      // the wave's sum(g^2): only lanes 0 and 32 hold non-zero values, so ssm_kernel's
-      // wave_sum_dpp_f64 adds exact zeros to them and equals (lane 0) + (lane 32)
-#pragma unroll
-      for (int j = 0; j < kTG; ++j) {
-        const double s = gsqd[j] + lane_plus32(gsqd[j]);  // (lane 0) + (lane 32) in lane 0
-        if (lane == 0 && t + j < nt) S.gpart[t + j][w] = s;
-      }
+      const double s = reduce4(acc[0], acc[1], acc[2], acc[3]);
+      if constexpr (W == 1) finish(s, k);
+      else S.part[w][4 * k + g][rl] = s;
     }
-    if (rd + 1 < rounds) scan_stage<PG>(buf[(rd + 1) & 1], raw, dtb, nA);
+    scan_stage<W, RB>(buf[(rd + 1) & 1], raw);
     lds_barrier();
-    // per-block sum(g^2) of this round's tokens, in ssm_kernel's order (waves 0 + 1 + 2 + 3)
-    if (tid < nt * PG) {
-      const int t = tid / PG, g = tid % PG;
-      const double* gp = &S.gpart[t][4 * g];
-      const int slot = head * (a.P / 16) + aa.pb0 + g;
-      a.sumsq_slots[((size_t)b * a.T + t0 + t) * a.n_slots + slot] = gp[0] + gp[1] + gp[2] + gp[3];
+    if constexpr (W > 1) {
+      // (the partials of a buffer are rewritten two rounds later, after the next round's barrier)
+      const int t = scan_item_token<W, RB>(0), i = scan_item_row<W, RB>();
+      double s = S.part[0][t][i] + S.part[1][t][i];
+      if constexpr (W == 4) s = s + (S.part[2][t][i] + S.part[3][t][i]);
+      finish(s, 0);
     }
   }
-  st_nt_f4(hp, f32x4{h0[0], h0[1], h0[2], h0[3]});
-  st_nt_f4(hp + 8 * a.N, f32x4{h1[0], h1[1], h1[2], h1[3]});
+#pragma unroll
+  for (int q = 0; q < NQ; ++q)
+    st_nt_f4(hp + 16 * (q < 4 ? Qa : Qb) + half + 4 * (q & 3), f32x4{h[4 * q], h[4 * q + 1], h[4 * q + 2], h[4 * q + 3]});
 }
 
 // dst[b] = src[b * T + T - 1]: the last token's row of every sequence.
@@ -291,25 +421,31 @@ __global__ __launch_bounds__(256) void last_rows_kernel(const uint16_t* __restri
   for (int k = threadIdx.x; k < D; k += 256) dst[(size_t)b * D + k] = s[k];
 }
 
-hipError_t launch_conv_seq(const ConvSeqArgs& a, int batch, hipStream_t s) {
-  hipLaunchKernelGGL(conv_seq_kernel, dim3((a.C + 255) / 256, batch), dim3(256), 0, s, a);
+hipError_t launch_conv_tokens(const ConvTokArgs& args, int batch, hipStream_t s) {
+  ConvTokArgs a = args;
+  if (a.T < 1 || batch < 1 || a.C % 8 || a.DI % 8 || a.ld % 8) return hipErrorInvalidValue;
+  // tokens per thread: 16 (the three re-read rows then cost 3/16 more) while that leaves 64 Ki
+  // threads (one wave per SIMD), else fewer, but
+  // at least the three tokens before any later range (only the first reads the conv state, which it writes)
+  a.tc = 16;
+  while (a.tc > 4 && (long long)batch * ((a.T + a.tc - 1) / a.tc) * (a.C / 8) < (1 << 16)) a.tc /= 2;
+  const dim3 g((a.C / 8 + 255) / 256 + 1, (a.T + a.tc - 1) / a.tc, batch);
+  hipLaunchKernelGGL(conv_tokens_kernel, g, dim3(256), 0, s, a);
   return hipGetLastError();
-}
-
-int scan_groups(int P) {
-  const int pbs = P / 16;
-  return pbs % 4 == 0 ? 4 : (pbs % 2 == 0 ? 2 : 1);
 }
 
 hipError_t launch_ssm_scan(const ScanArgs& a, int batch, hipStream_t s) {
   if (a.T < 1 || a.P % 16 || a.N != 128) return hipErrorInvalidValue;
-  const int PG = scan_groups(a.P);
-  const dim3 grid(a.H * (a.P / (16 * PG)), batch);
-  switch (PG) {
-    case 4: hipLaunchKernelGGL(ssm_scan_kernel<4>, grid, dim3(1024), 0, s, a); break;
-    case 2: hipLaunchKernelGGL(ssm_scan_kernel<2>, grid, dim3(512), 0, s, a); break;
-    default: hipLaunchKernelGGL(ssm_scan_kernel<1>, grid, dim3(256), 0, s, a); break;
-  }
+  // Waves per 16-row block: the fewest that leave two waves per SIMD (2048 on the chip), where the
+  // head has enough blocks for a workgroup of four waves
+  const int blocks = a.P / 16;
+  const long long waves = (long long)batch * a.H * blocks;
+  if (blocks % 4 == 0 && waves >= 2048)
+    hipLaunchKernelGGL((ssm_scan_kernel<1, 4>), dim3(a.H * (blocks / 4), batch), dim3(256), 0, s, a);
+  else if (blocks % 2 == 0 && 2 * waves >= 2048)
+    hipLaunchKernelGGL((ssm_scan_kernel<2, 2>), dim3(a.H * (blocks / 2), batch), dim3(256), 0, s, a);
+  else
+    hipLaunchKernelGGL((ssm_scan_kernel<4, 1>), dim3(a.H * blocks, batch), dim3(256), 0, s, a);
   return hipGetLastError();
 }
 

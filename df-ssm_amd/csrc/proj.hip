@@ -203,7 +203,6 @@ __global__ __launch_bounds__(kPT) void prep_kernel(PrepArgs a, int M) {
 constexpr int kPrepRows = 16;
 constexpr int kPrepRowsT = kMaxK / 8;  // threads per workgroup at most
 
-template <int MODE>
 __global__ __launch_bounds__(kPrepRowsT) void prep_rows_kernel(PrepArgs a, int M) {
   __shared__ double red_d[kPrepRowsT / 64];
   __shared__ double red_h[kPrepRowsT / 64][DFSSM_LORA_R];
@@ -213,15 +212,8 @@ __global__ __launch_bounds__(kPrepRowsT) void prep_rows_kernel(PrepArgs a, int M
   const int K = a.K, nw = (int)blockDim.x >> 6;
   const int m0 = (int)blockIdx.x * kPrepRows, m1 = m0 + kPrepRows < M ? m0 + kPrepRows : M;
   const bool want_sum = a.s_out != nullptr;
-  // this row's activations (and its sum-of-squares slot) are loaded one row ahead
-  auto load_row = [&](int m, u32x4& av, double& slot) {
-    const int mm = m < m1 ? m : m1 - 1;
-    av = *(const u32x4*)(a.act + (size_t)mm * a.ld_act + 8 * tid);
-    if (MODE == DFSSM_MODE_OUT) slot = a.sumsq_slots[(size_t)mm * a.n_slots + (tid < a.n_slots ? tid : a.n_slots - 1)];
-  };
-  u32x4 av;
-  double slot = 0.0;
-  load_row(m0, av, slot);
+  // this row's activations are loaded one row ahead
+  u32x4 av = *(const u32x4*)(a.act + (size_t)m0 * a.ld_act + 8 * tid);
   const f32x4 w0 = *(const f32x4*)(a.norm_w + 8 * tid);
   const f32x4 w1 = *(const f32x4*)(a.norm_w + 8 * tid + 4);
   const float wv[8] = {w0[0], w0[1], w0[2], w0[3], w1[0], w1[1], w1[2], w1[3]};
@@ -251,17 +243,12 @@ __global__ __launch_bounds__(kPrepRowsT) void prep_rows_kernel(PrepArgs a, int M
 #pragma unroll
       for (int j = 0; j < 4; ++j) asm volatile("" : "+v"(bp[rr][j]));
     const u32x4 cur = av;
-    const double cslot = slot;
-    if (m + 1 < m1) load_row(m + 1, av, slot);
+    if (m + 1 < m1) av = *(const u32x4*)(a.act + (size_t)(m + 1) * a.ld_act + 8 * tid);
     double part = 0.0;
-    if (MODE == DFSSM_MODE_IN) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const double xv = (double)h2f((uint16_t)(cur[e >> 1] >> (16 * (e & 1))));
-        part += xv * xv;
-      }
-    } else {
-      part = tid < a.n_slots ? cslot : 0.0;
+    for (int e = 0; e < 8; ++e) {
+      const double xv = (double)h2f((uint16_t)(cur[e >> 1] >> (16 * (e & 1))));
+      part += xv * xv;
     }
     {
       const double pw = wave_sum_dpp_f64(part);
@@ -962,14 +949,11 @@ hipError_t launch_prep(const PrepArgs& a, int M, int mode, hipStream_t s) {
   if (mode == DFSSM_MODE_OUT && (!a.sumsq_slots || a.n_slots < 1 || a.n_slots > a.K / 8)) return hipErrorInvalidValue;
   if (a.lB && !a.lBs) return hipErrorInvalidValue;
   if (a.K > kMaxK || a.K % 512) return hipErrorInvalidValue;  // K / 8 threads: whole waves
-  const bool rows_path = M > 64 && !a.planes_out && !a.xn_out && !a.xs16_out && (a.h_out || !a.lB);
+  const bool rows_path = mode == DFSSM_MODE_IN && M > 64 && !a.planes_out && !a.xn_out && !a.xs16_out && (a.h_out || !a.lB);
   if (a.q_tiled && !rows_path) return hipErrorInvalidValue;
   if (rows_path) {  // many rows: one pass each
     const dim3 g((M + kPrepRows - 1) / kPrepRows);
-    if (mode == DFSSM_MODE_IN)
-      hipLaunchKernelGGL(prep_rows_kernel<DFSSM_MODE_IN>, g, dim3(a.K / 8), 0, s, a, M);
-    else
-      hipLaunchKernelGGL(prep_rows_kernel<DFSSM_MODE_OUT>, g, dim3(a.K / 8), 0, s, a, M);
+    hipLaunchKernelGGL(prep_rows_kernel, g, dim3(a.K / 8), 0, s, a, M);
     return hipGetLastError();
   }
   // 16 workgroups of K / 8 threads per row while they are all resident at once (at most 32 waves

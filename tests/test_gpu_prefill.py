@@ -113,3 +113,36 @@ def test_prefill_rejects_bad_prompts(tiny_weights):
         gpu.prefill(torch.zeros(3, 4, dtype=torch.int64))
     with pytest.raises(IndexError):
         gpu.prefill(torch.full((2, 4), tiny_weights.cfg.vocab_size, dtype=torch.int64))
+
+
+@pytest.mark.parametrize("B,T,heads,headdim", [(5, 18, 16, 64), (5, 4, 16, 64), (17, 9, 16, 64), (24, 7, 32, 32),
+                                               (32, 13, 16, 64), (40, 1, 16, 64), (64, 5, 64, 16)])
+def test_prefill_readout_order(B, T, heads, headdim):
+    """The scan's C.h sums are added in the order of the batched decode step, in each of its forms (four,
+    two and one waves per 16-row block: B * 1024 / 16 blocks on a chip of 1024 SIMDs). A state of large
+    values that cancel in pairs (C constant, B zero) makes every fp64 sum depend on its order, by far
+    more than the fp16 rounding of y."""
+    c = DFSSMConfig(n_layer=1, d_model=512, d_inner=1024, d_state=128, nheads=heads, headdim=headdim, ngroups=1,
+                    vocab_size=1000, kw=4)
+    w = make_weights(c, seed=3)
+    L = w.layers[0]
+    L["conv_w"][1024:] = 0
+    L["conv_b"][1024:1152] = 0          # B = silu(0) = 0
+    L["conv_b"][1152:] = 1.5            # C = one constant
+    rng = np.random.default_rng(4)
+    P = headdim
+    big = (rng.uniform(1, 2, (B, heads, P, 32)) * 2.0 ** 50).astype(np.float32)
+    h = np.concatenate([big, -big, rng.normal(0, 1, (B, heads, P, 64)).astype(np.float32)], axis=-1)
+    h = np.take_along_axis(h, rng.permuted(np.tile(np.arange(128), (B, heads, P, 1)), axis=-1), axis=-1)
+    # the sum does depend on the order: 64-bit sums of two orders differ by more than fp16 resolves
+    d = h.astype(np.float64)
+    assert np.median(np.abs(d.cumsum(-1)[..., -1] - d[..., ::-1].cumsum(-1)[..., -1])) > 0.01
+    print(f"readout order B={B} T={T} {heads} x {headdim}", flush=True)
+    pf, st = _twins(w, B)
+    for m in (pf, st):
+        m.h_state[0].copy_(torch.from_numpy(h))
+    prompts = torch.from_numpy(make_prompts(B, c.vocab_size, T))
+    lp = pf.prefill(prompts, want_logits=True)
+    st.ingest(prompts[:, :-1], step_by_step=True)
+    ls = st.forward(prompts[:, -1].to(DEV))
+    _assert_same(pf, st, lp, ls)
