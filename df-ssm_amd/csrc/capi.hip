@@ -717,6 +717,7 @@ static int prefill_chunk(const dfssm_model* model, const int64_t* tokens, int n_
       p.norm_w = in ? Lw.ln_w : Lw.norm_w;
       p.lB = in ? Lw.in_lB : Lw.out_lB;
       p.lBs = in ? Lw.in_lB_s : Lw.out_lB_s;
+      p.lBq = in ? Lw.in_lBq : Lw.out_lBq;
       p.q_out = (int8_t*)(pw + w.q);
       p.ld_q = kq;
       p.xs_out = (float*)(pw + w.xs);

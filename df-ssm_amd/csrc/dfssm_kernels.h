@@ -20,6 +20,7 @@ struct PrepArgs {
   int n_slots;
   const int8_t* lB;          // (16, K) LoRA B, int8 (null: no LoRA intermediate)
   const uint16_t* lBs;       // (16) fp16
+  const uint16_t* lBq;       // (16, K) fp16(lB lBs), 16-byte aligned: the many-row path's LoRA B
   int8_t* q_out;             // (M, ld_q) int8 activations, or null
   uint32_t* planes_out;      // (M, ld_q/32, 8) bit planes of q, or null
   int ld_q;
@@ -92,6 +93,7 @@ struct GemmPro {
   const float* norm_w;       // (N) fp32 RMSNorm weight of the next layer
   const int8_t* lB;          // (16, N) its LoRA B, int8 (null: no LoRA intermediate)
   const uint16_t* lBs;       // (16) fp16
+  const uint16_t* lBq;       // (16, K) fp16(lB lBs), 16-byte aligned: the many-row path's LoRA B
   int8_t* q_out;             // (M, ld_q) int8 activations
   int ld_q;
   float* xs_out;             // (M) activation scale (an fp16 value)
@@ -172,6 +174,7 @@ struct SsmPrepArgs {
   const float* norm_w;       // (H P) fp32 gated-RMSNorm weight
   const int8_t* lB;          // (16, H P) LoRA B, int8 (null: no LoRA intermediate)
   const uint16_t* lBs;       // (16) fp16
+  const uint16_t* lBq;       // (16, K) fp16(lB lBs), 16-byte aligned: the many-row path's LoRA B
   int8_t* q_out;             // (M, ld_q) int8 activations
   int ld_q;
   float* xs_out;             // (M) activation scale (an fp16 value)

@@ -192,131 +192,137 @@ __global__ __launch_bounds__(kPT) void prep_kernel(PrepArgs a, int M) {
   }
 }
 
-// prep_rows_kernel: the same prologue for many rows (the prompt prefill runs thousands), one
-// workgroup of K/8 threads per kPrepRows consecutive rows. The norm weights and the fp16 LoRA-B
-// values of a thread's 8 columns (16 ranks) stay in registers across the rows, and each row's
-// RMSNorm, quantizer and 16 LoRA intermediates are computed once (prep_kernel's 16 workgroups per
-// row each recompute the norm). The thread -> column map, the per-thread order of the fp64 sums
-// and the reduction trees are prep_kernel's, so every output is identical. Writes q_out (row-major
-// or, with q_tiled, in the wide GEMM's tiled layout), xs_out, h_out and s_out; the decode-only
-// outputs (planes_out, xn_out, xs16_out) are not supported.
-constexpr int kPrepRows = 16;
-constexpr int kPrepRowsT = kMaxK / 8;  // threads per workgroup at most
+// ------------------------------------------------------------------------------------------
+// prep_rows_kernel<K / 512>: the same prologue for many rows (the prompt prefill runs thousands), one
+// workgroup of 16 waves per 16 rows. Wave w has row w in registers for the RMSNorm, the maximum and
+// the quantizer (no exchange between waves); the 16 x 16 LoRA intermediates of the workgroup are one
+// contraction over K and run on the fp64 matrix cores (v_mfma_f64_16x16x4f64: exact products of fp16
+// values, fp64 sums): the normalized rows go through LDS, up to 2560 columns at a time, each wave
+// takes 32 columns of every 512 and the waves' sums are added through LDS. Within an MFMA step lane
+// group g supplies column 8 g + s of a 32-column block for both operands (a permutation of k), so
+// both come as 16-byte vectors. With q_tiled the 16 rows of q are one contiguous block of the wide
+// GEMM's layout: staged in LDS (16-byte units, swizzled by their 16-column block: a row's units are 256
+// bytes apart) and stored as one. The decode-only outputs are not supported.
+//
+// What bounds it: VALU issue (about 18 instructions per value) and the fp64 matrix rate, both about
+// 9 us per workgroup at K = 5120, one workgroup per CU. Measured against one workgroup of K / 8 threads
+// walking 16 rows one after the other (a row's 16 ranks as fp64 fmas and wave reductions): 497 -> 123
+// us at 16 384 rows of K = 5120, 337 -> 65 us at K = 2560, 89 -> 22 and 67 -> 13 us at 999 rows of K =
+// 4096 and 2048 (63 workgroups: one round).
+// ------------------------------------------------------------------------------------------
+constexpr int kPrepRowsT = 1024;
+typedef double prep_v4d __attribute__((ext_vector_type(4)));
 
+template <int KB>
 __global__ __launch_bounds__(kPrepRowsT) void prep_rows_kernel(PrepArgs a, int M) {
-  __shared__ double red_d[kPrepRowsT / 64];
-  __shared__ double red_h[kPrepRowsT / 64][DFSSM_LORA_R];
-  __shared__ float red_f[kPrepRowsT / 64];
-  __shared__ int red_i[kPrepRowsT / 64];
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int K = a.K, nw = (int)blockDim.x >> 6;
-  const int m0 = (int)blockIdx.x * kPrepRows, m1 = m0 + kPrepRows < M ? m0 + kPrepRows : M;
-  const bool want_sum = a.s_out != nullptr;
-  // this row's activations are loaded one row ahead
-  u32x4 av = *(const u32x4*)(a.act + (size_t)m0 * a.ld_act + 8 * tid);
-  const f32x4 w0 = *(const f32x4*)(a.norm_w + 8 * tid);
-  const f32x4 w1 = *(const f32x4*)(a.norm_w + 8 * tid + 4);
-  const float wv[8] = {w0[0], w0[1], w0[2], w0[3], w1[0], w1[1], w1[2], w1[3]};
-  // fp16(B_i8 * B_s) of the 8 columns for every rank, as fp16 pairs (prep_kernel's b0, b1)
-  uint32_t bp[DFSSM_LORA_R][4];
+  constexpr int K = 512 * KB;
+  constexpr int PC = KB <= 5 ? KB : (KB + 1) / 2;  // 512-column chunks per LoRA pass
+  constexpr int XS = PC * 1024 + 16;               // LDS bytes of a row of a pass (padded)
+  constexpr int kLds = 16 * XS > 16 * K ? (16 * XS > 32768 ? 16 * XS : 32768) : (16 * K > 32768 ? 16 * K : 32768);
+  __shared__ __attribute__((aligned(16))) uint8_t lds[kLds];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int m0 = (int)blockIdx.x * 16, m = m0 + w;
+  const bool live = m < M;  // (rows past the end recompute the last one and store nothing but padding)
+  const uint16_t* act = a.act + (size_t)(live ? m : M - 1) * a.ld_act + 8 * lane;
+  u32x4 v[KB];
 #pragma unroll
-  for (int rr = 0; rr < DFSSM_LORA_R; ++rr) {
-    uint2 b8 = {0u, 0u};
-    float bs = 0.0f;
-    if (a.lB) {
-      b8 = *(const uint2*)(a.lB + (size_t)rr * K + 8 * tid);
-      bs = h2f(a.lBs[rr]);
+  for (int j = 0; j < KB; ++j) v[j] = *(const u32x4*)(act + 512 * j);
+  double part = 0.0;
+#pragma unroll
+  for (int j = 0; j < KB; ++j)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const double x = (double)h2f((uint16_t)(v[j][e >> 1] >> (16 * (e & 1))));
+      part = __builtin_fma(x, x, part);  // (x x is exact)
     }
-    const uint32_t bw[2] = {b8.x, b8.y};
+  const float var = (float)wave_sum_dpp_f64(part) * (1.0f / (float)K);
+  const float r = 1.0f / sqrt_rn(var + 1e-5f);
+  float mx = 0.0f;
+#pragma unroll
+  for (int j = 0; j < KB; ++j) {
+    const f32x4 w0 = *(const f32x4*)(a.norm_w + 512 * j + 8 * lane);
+    const f32x4 w1 = *(const f32x4*)(a.norm_w + 512 * j + 8 * lane + 4);
+    const float wv[8] = {w0[0], w0[1], w0[2], w0[3], w1[0], w1[1], w1[2], w1[3]};
 #pragma unroll
     for (int e = 0; e < 8; e += 2) {
-      const float b0 = r16((float)(int8_t)(bw[e >> 2] >> (8 * (e & 3))) * bs);
-      const float b1 = r16((float)(int8_t)(bw[(e + 1) >> 2] >> (8 * ((e + 1) & 3))) * bs);
-      bp[rr][e >> 1] = (uint32_t)f2h(b0) | ((uint32_t)f2h(b1) << 16);
+      const uint32_t x2 = v[j][e >> 1];
+      const float x0 = r16((h2f((uint16_t)x2) * r) * wv[e]);
+      const float x1 = r16((h2f((uint16_t)(x2 >> 16)) * r) * wv[e + 1]);
+      mx = fmaxf(mx, fmaxf(fabsf(x0), fabsf(x1)));
+      v[j][e >> 1] = (uint32_t)f2h(x0) | ((uint32_t)f2h(x1) << 16);
     }
   }
-  for (int m = m0; m < m1; ++m) {
-    // opaque per row: keeps the 128 conversions of bp to fp32 inside the loop (hoisted, they
-    // would not fit the registers)
+  const float xs = quant_scale(wave_max_dpp_f32(mx));
+  const float rinv = quant_rcp(xs);
+  // this lane's LoRA-B vectors of the first pass, under the quantizer
+  const int li = lane & 15, g = lane >> 4;
+  const uint16_t* lb = a.lBq + (size_t)li * K + 32 * w + 8 * g;
+  u32x4 bv[PC];
 #pragma unroll
-    for (int rr = 0; rr < DFSSM_LORA_R; ++rr)
+  for (int j = 0; j < PC; ++j) bv[j] = *(const u32x4*)(lb + 512 * j);
+  asm volatile("" ::: "memory");  // issued here, not sunk to their use
+  if (live && lane == 0 && a.xs_out) a.xs_out[m] = xs;
+  if (a.q_out) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) asm volatile("" : "+v"(bp[rr][j]));
-    const u32x4 cur = av;
-    if (m + 1 < m1) av = *(const u32x4*)(a.act + (size_t)(m + 1) * a.ld_act + 8 * tid);
-    double part = 0.0;
+    for (int j = 0; j < KB; ++j) {
+      uint32_t qw[2] = {0u, 0u};
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const double xv = (double)h2f((uint16_t)(cur[e >> 1] >> (16 * (e & 1))));
-      part += xv * xv;
-    }
-    {
-      const double pw = wave_sum_dpp_f64(part);
-      if (lane == 0) red_d[w] = pw;
-    }
-    lds_barrier();
-    double ss = 0.0;
-    for (int i = 0; i < nw; ++i) ss += red_d[i];
-    const float var = (float)ss * (1.0f / (float)K);
-    const float r = 1.0f / sqrt_rn(var + 1e-5f);
-    float xn[8];
-    float mx = 0.0f;
-#pragma unroll
-    for (int e = 0; e < 8; e += 2) {
-      xn[e] = r16((h2f((uint16_t)(cur[e >> 1])) * r) * wv[e]);
-      xn[e + 1] = r16((h2f((uint16_t)(cur[e >> 1] >> 16)) * r) * wv[e + 1]);
-      mx = fmaxf(mx, fmaxf(fabsf(xn[e]), fabsf(xn[e + 1])));
-    }
-    {
-      const float mw = wave_max_dpp_f32(mx);
-      if (lane == 0) red_f[w] = mw;
-    }
-#pragma unroll
-    for (int rr = 0; rr < DFSSM_LORA_R; ++rr) {  // one rank at a time: columns in order, as prep_kernel
-      double hacc = 0.0;
-#pragma unroll
-      for (int e = 0; e < 8; e += 2) {  // fp16 x fp16 is exact in fp32
-        hacc += (double)(xn[e] * h2f((uint16_t)bp[rr][e >> 1]));
-        hacc += (double)(xn[e + 1] * h2f((uint16_t)(bp[rr][e >> 1] >> 16)));
+      for (int e = 0; e < 8; ++e) {
+        const int q = quant_i8(h2f((uint16_t)(v[j][e >> 1] >> (16 * (e & 1)))), rinv);
+        qw[e >> 2] |= (uint32_t)(q & 0xff) << (8 * (e & 3));
       }
-      const double hw = wave_sum_dpp_f64(hacc);
-      if (lane == 0) red_h[w][rr] = hw;
+      const uint2 qv = {qw[0], qw[1]};
+      if (a.q_tiled) {
+        const int blk = 32 * j + (lane >> 1);  // 16-column block; this lane's half of it
+        *(uint2*)&lds[256 * blk + 16 * (w ^ (blk & 15)) + 8 * (lane & 1)] = qv;
+      } else if (live) {
+        *(uint2*)(a.q_out + (size_t)m * a.ld_q + 512 * j + 8 * lane) = qv;
+      }
     }
-    lds_barrier();  // (every wave has also read red_d: the next row may rewrite it)
-    float amax = red_f[0];
-    for (int i = 0; i < nw; ++i) amax = fmaxf(amax, red_f[i]);
-    if (a.lB && tid < DFSSM_LORA_R) {
-      double ht = 0.0;
-      for (int i = 0; i < nw; ++i) ht += red_h[i][tid];
-      a.h_out[(size_t)m * DFSSM_LORA_R + tid] = r16((float)ht);
-    }
-    const float xs = quant_scale(amax);
-    const float rinv = quant_rcp(xs);
-    uint32_t qw[2] = {0u, 0u};
-    int qsum = 0;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int q = quant_i8(xn[e], rinv);
-      qsum += q;
-      qw[e >> 2] |= (uint32_t)(q & 0xff) << (8 * (e & 3));
-    }
-    if (a.q_out) {
-      int8_t* qp = a.q_tiled ? a.q_out + wide_tiled_offset(m, 8 * tid, K) : a.q_out + (size_t)m * a.ld_q + 8 * tid;
-      *(uint2*)qp = uint2{qw[0], qw[1]};
-    }
-    int S = 0;
-    if (want_sum) {  // uniform
-      const int qs = wave_sum_dpp_i32(qsum);
-      if (lane == 0) red_i[w] = qs;
+    if (a.q_tiled) {
       lds_barrier();
-      for (int i = 0; i < nw; ++i) S += red_i[i];
+      u32x4* qt = (u32x4*)(a.q_out + (size_t)m0 * K);  // the 16 rows of the tile
+      for (int u = tid; u < K; u += kPrepRowsT) {      // 16-byte units [blk][row]
+        const int blk = u >> 4, row = u & 15;
+        qt[u] = *(const u32x4*)&lds[256 * blk + 16 * (row ^ (blk & 15))];
+      }
+      lds_barrier();
     }
-    if (tid == 0) {
-      if (a.s_out) a.s_out[m] = S;
-      if (a.xs_out) a.xs_out[m] = xs;
+  }
+  prep_v4d acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int j0 = 0; j0 < KB; j0 += PC) {
+    if (j0) {
+#pragma unroll
+      for (int j = j0; j < KB; ++j) bv[j - j0] = *(const u32x4*)(lb + 512 * j);
+      asm volatile("" ::: "memory");
+      lds_barrier();  // every wave has read the previous pass
     }
-    // red_f and red_h are rewritten only after the next row's first barrier, red_i after its
-    // second: every wave has read them by then
+#pragma unroll
+    for (int j = j0; j < KB && j < j0 + PC; ++j) *(u32x4*)&lds[w * XS + (j - j0) * 1024 + 16 * lane] = v[j];
+    lds_barrier();
+#pragma unroll
+    for (int j = j0; j < KB && j < j0 + PC; ++j) {
+      const u32x4 av = *(const u32x4*)&lds[li * XS + (j - j0) * 1024 + 2 * (32 * w + 8 * g)];
+      const u32x4 b = bv[j - j0];
+#pragma unroll
+      for (int s = 0; s < 8; ++s)
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)h2f((uint16_t)(av[s >> 1] >> (16 * (s & 1)))),
+                                                   (double)h2f((uint16_t)(b[s >> 1] >> (16 * (s & 1)))), acc, 0, 0, 0);
+    }
+  }
+  lds_barrier();  // every wave has read the last pass
+  double* part_h = (double*)lds;  // [wave][i][lane]: row lane / 16 + 4 i, rank lane % 16
+#pragma unroll
+  for (int i = 0; i < 4; ++i) part_h[w * 256 + 64 * i + lane] = acc[i];
+  lds_barrier();
+  if (tid < 256) {
+    double h = 0.0;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) h += part_h[256 * i + tid];
+    const int row = m0 + ((tid & 63) >> 4) + 4 * (tid >> 6);
+    if (row < M) a.h_out[(size_t)row * DFSSM_LORA_R + (tid & 15)] = r16((float)h);
   }
 }
 
@@ -949,11 +955,20 @@ hipError_t launch_prep(const PrepArgs& a, int M, int mode, hipStream_t s) {
   if (mode == DFSSM_MODE_OUT && (!a.sumsq_slots || a.n_slots < 1 || a.n_slots > a.K / 8)) return hipErrorInvalidValue;
   if (a.lB && !a.lBs) return hipErrorInvalidValue;
   if (a.K > kMaxK || a.K % 512) return hipErrorInvalidValue;  // K / 8 threads: whole waves
-  const bool rows_path = mode == DFSSM_MODE_IN && M > 64 && !a.planes_out && !a.xn_out && !a.xs16_out && (a.h_out || !a.lB);
+  // many rows: prep_rows_kernel
+  const bool rows_path = mode == DFSSM_MODE_IN && M > 64 && a.lBq && a.h_out && !a.planes_out && !a.xn_out &&
+                         !a.xs16_out && !a.s_out;
   if (a.q_tiled && !rows_path) return hipErrorInvalidValue;
-  if (rows_path) {  // many rows: one pass each
-    const dim3 g((M + kPrepRows - 1) / kPrepRows);
-    hipLaunchKernelGGL(prep_rows_kernel, g, dim3(a.K / 8), 0, s, a, M);
+  if (rows_path) {
+    const dim3 g((M + 15) / 16);
+    switch (a.K / 512) {
+#define DFSSM_PREP_KB(kb) \
+  case kb: hipLaunchKernelGGL((prep_rows_kernel<kb>), g, dim3(kPrepRowsT), 0, s, a, M); break;
+      DFSSM_PREP_KB(1) DFSSM_PREP_KB(2) DFSSM_PREP_KB(3) DFSSM_PREP_KB(4) DFSSM_PREP_KB(5)
+      DFSSM_PREP_KB(6) DFSSM_PREP_KB(7) DFSSM_PREP_KB(8) DFSSM_PREP_KB(9) DFSSM_PREP_KB(10)
+#undef DFSSM_PREP_KB
+      default: return hipErrorInvalidValue;
+    }
     return hipGetLastError();
   }
   // 16 workgroups of K / 8 threads per row while they are all resident at once (at most 32 waves

@@ -107,6 +107,16 @@ def test_prefill_2p7b_layer_shapes():
     _prefill_vs_steps(w, 64, 20)
 
 
+@pytest.mark.parametrize("dm,di,B,T", [(1536, 3072, 5, 27), (1536, 3072, 7, 41), (512, 3584, 9, 29), (4608, 512, 6, 43)])
+def test_prefill_many_rows(dm, di, B, T):
+    """The many-row prologue (more than 64 rows) at odd multiples of 512 columns, one and two passes of
+    the LoRA contraction, row counts no tile divides, q row-major (under 256 rows) and tiled."""
+    c = DFSSMConfig(n_layer=2, d_model=dm, d_inner=di, d_state=128, nheads=di // 64, headdim=64, ngroups=1,
+                    vocab_size=1000, kw=4)
+    print(f"prefill rows {B * T} of {dm} / {di}", flush=True)
+    _prefill_vs_steps(make_weights(c, seed=11), B, T)
+
+
 def test_prefill_rejects_bad_prompts(tiny_weights):
     gpu = DFSSMModel.from_weights(tiny_weights, device=DEV, batch_size=2)
     with pytest.raises(ValueError):
