@@ -79,11 +79,12 @@ WsLayout ws_layout(const dfssm_dims* d) {
 // residual stream of every row, the projection rows, g, the sum(g^2) slots and the prologue
 // outputs (q, scale, LoRA intermediate).
 struct PfLayout {
-  size_t x, proj, g, bc, dec, q, xs, h, w8, total;
+  size_t x, proj, g, bc, dec, q, qs, xs, h, total;
 };
-// Prefill chunks of at least this many rows run the projections on the wide GEMM (weights
-// expanded to int8 in the prefill workspace), smaller ones on gemm_kernel.
-constexpr int kWideGemmRows = 256;
+// Prefill chunks of at least this many rows run the many-row prologue and the wide GEMM, smaller ones
+// the decode kernels, which take 64 rows. At 80 rows the two projections cost the same (1.3B: 22.6 us
+// on gemm_kernel, 23.7 here; 2.7B: 29.2 and 27.2), at 128 they cost 30.8 and 23.9 us (1.3B).
+constexpr int kWideGemmRows = 65;
 
 PfLayout pf_layout(const Derived& r, int rows) {
   PfLayout w;
@@ -95,13 +96,9 @@ PfLayout pf_layout(const Derived& r, int rows) {
   w.bc = off;    off = align_up(off + (size_t)rows * 2 * r.N * 2);
   w.dec = off;   off = align_up(off + (size_t)rows * r.H * 8);
   w.q = off;     off = align_up(off + (size_t)(rows + 15) / 16 * 16 * kq);  // rows padded to 16 (tiled)
+  w.qs = off;    off = align_up(off + (size_t)rows * 4);
   w.xs = off;    off = align_up(off + (size_t)rows * 4);
   w.h = off;     off = align_up(off + (size_t)rows * 16 * 4);
-  w.w8 = off;
-  if (rows >= kWideGemmRows) {  // the larger projection's expanded weights
-    const size_t a = gemm_wide_w8_bytes(r.IPO, r.D), b = gemm_wide_w8_bytes(r.D, r.DI);
-    off = align_up(off + (a > b ? a : b));
-  }
   w.total = off;
   return w;
 }
@@ -723,12 +720,14 @@ static int prefill_chunk(const dfssm_model* model, const int64_t* tokens, int n_
       p.xs_out = (float*)(pw + w.xs);
       p.h_out = (float*)(pw + w.h);
       p.K = in ? r.D : r.DI;
-      p.q_tiled = R >= kWideGemmRows;  // the wide GEMM reads q tiled
+      p.q_tiled = R >= kWideGemmRows;
+      p.s_out = p.q_tiled ? (int*)(pw + w.qs) : nullptr;
       st = launch_prep(p, R, DFSSM_MODE_IN, s);  // (sum(g^2) from the row itself)
       if (st != hipSuccess) return hip_status(st);
       GemmArgs a{};
       a.q = (const int8_t*)(pw + w.q); a.ld_q = kq; a.M = R;
       a.xs = (const float*)(pw + w.xs);
+      a.qsum = (const int*)(pw + w.qs);
       a.h = (const float*)(pw + w.h);
       if (in) {  // raw projection rows: the conv runs over the tokens below
         a.bits = Lw.in_bits; a.wscale = Lw.in_scale; a.lA = Lw.in_lA; a.lAs = Lw.in_lA_s;
@@ -739,7 +738,7 @@ static int prefill_chunk(const dfssm_model* model, const int64_t* tokens, int n_
         a.out = xr; a.ld_out = r.D;
         a.N = r.D; a.K = r.DI;
       }
-      st = R >= kWideGemmRows ? launch_gemm_wide(a, in ? DFSSM_MODE_IN : DFSSM_MODE_OUT, (int8_t*)(pw + w.w8), s)
+      st = R >= kWideGemmRows ? launch_gemm_wide(a, in ? DFSSM_MODE_IN : DFSSM_MODE_OUT, s)
                               : launch_gemm(a, in ? DFSSM_MODE_IN : DFSSM_MODE_OUT, s);
       if (st != hipSuccess) return hip_status(st);
       if (!in) break;

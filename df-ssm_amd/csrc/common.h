@@ -227,6 +227,17 @@ __device__ __forceinline__ int quant_i8(float x, float r) {
   return (int)__builtin_amdgcn_fmed3f(t, -128.0f, 127.0f);
 }
 
+// Within each quad of lanes (4i..4i+3, quad lane b = lane % 4): byte j of the result of lane b is
+// byte b of lane j's a (a 4 x 4 byte transpose: two DPP quad permutations and two byte selects).
+// v_perm_b32 (src0, src1, sel): byte k of the result is byte sel_k of the 8 bytes
+// {src1 bytes 0..3, src0 bytes 0..3}.
+__device__ __forceinline__ uint32_t quad_transpose_bytes(uint32_t a, int b) {
+  const uint32_t p = (uint32_t)dpp_i32<0x4E>((int)a);  // lane b ^ 2
+  const uint32_t u = __builtin_amdgcn_perm(p, a, (b & 2) ? 0x03020706u : 0x05040100u);
+  const uint32_t q = (uint32_t)dpp_i32<0xB1>((int)u);  // lane b ^ 1
+  return __builtin_amdgcn_perm(q, u, (b & 1) ? 0x03070105u : 0x06020400u);
+}
+
 // Bit planes of 64 int8 values, one per lane (q of element k0 + lane): w[b] = bit b of elements
 // k0 .. k0 + 31, w[8 + b] = bit b of elements k0 + 32 .. k0 + 63 (one ballot per plane). The
 // words are wave-uniform (scalar registers); one lane stores them (planes_store).

@@ -24,21 +24,20 @@ struct PrepArgs {
   int8_t* q_out;             // (M, ld_q) int8 activations, or null
   uint32_t* planes_out;      // (M, ld_q/32, 8) bit planes of q, or null
   int ld_q;
-  int* s_out;                // (M) sum of q
+  int* s_out;                // (M) sum of q, or null
   float* xs_out;             // (M) activation scale (an fp16 value)
   float* h_out;              // (M, 16) LoRA intermediate (fp16 values)
   uint16_t* xn_out;          // (M, K) normalized activations, or null
   uint16_t* xs16_out;        // (M) activation scale as fp16 bits, or null
   int K;
-  int q_tiled;               // q_out in the 16-row tiled layout of the wide GEMM (many-row path only)
+  int q_tiled;               // many rows: q_out (and all of q, s, xs, h) for the wide GEMM, in its layout
 };
-// The wide GEMM's operand layout (activations q and expanded weights): 16-row tiles of 64-column
-// k steps, [row / 16][k / 64][(k / 16) % 4][row % 16][k % 16], so that lane l of a wave reading
-// (row tile, k step) takes bytes 16 l .. 16 l + 15: one contiguous 1 KiB per wave-wide load.
-// K is a multiple of 64; the rows are padded to a multiple of 16.
-__host__ __device__ inline size_t wide_tiled_offset(int row, int k, int K) {
-  return (((size_t)(row >> 4) * (K >> 6) + (k >> 6)) * 4 + ((k >> 4) & 3)) * 256 + (row & 15) * 16 + (k & 15);
-}
+// The wide GEMM's activation layout: 16-row tiles of 64-column k steps, 1 KiB each, [row / 16][k step]
+// [g][row % 16][16 bytes], so that lane (g, row) of a wave takes 16 contiguous bytes of a contiguous
+// KiB. Step 8 j + s holds, as bytes 4 d + b of group g, the columns 512 j + 128 g + 32 d + 8 b + s: bit
+// 8 b + s of word d of the sign-bit chunk 4 j + g, so the lanes of group g make the other operand from
+// one chunk each, four bytes at a time: (word >> s) & 0x01010101.
+constexpr int kWideTile = 16;  // rows of a tile (the buffer is padded to whole tiles)
 
 struct ProjArgs {
   const uint32_t* bits;      // tiled sign bits [N_pad/64][K/128][64][4]
@@ -70,6 +69,7 @@ struct GemmArgs {
   const int8_t* q;           // (M, ld_q) int8 activations
   int ld_q, M;
   const float* xs;           // (M) activation scales (fp16 values) or null
+  const int* qsum;           // (M) row sums of q (wide GEMM)
   const uint16_t* xs16;      // (M) fp16 activation scales (SCAFFOLD), used when xs is null
   const float* h;            // (M, 16) LoRA intermediate (IN / OUT)
   const uint16_t* h16;       // SCAFFOLD with LoRA (lA non-null): (M, 16) fp16 intermediates
@@ -82,7 +82,7 @@ struct GemmArgs {
   int conv_lo, conv_c;
   int N, K;
 };
-constexpr int kGemmMaxRows = 32768;
+constexpr int kGemmMaxRows = 32768;  // wide GEMM
 // Decode at batch >= 5: the next layer's in_proj prologue (prep_kernel<IN>'s outputs) computed
 // by M extra workgroups of the out_proj launch, after every GEMM workgroup, from the new x rows
 // handed over as tagged words (tag << 16) | fp16.
@@ -93,7 +93,6 @@ struct GemmPro {
   const float* norm_w;       // (N) fp32 RMSNorm weight of the next layer
   const int8_t* lB;          // (16, N) its LoRA B, int8 (null: no LoRA intermediate)
   const uint16_t* lBs;       // (16) fp16
-  const uint16_t* lBq;       // (16, K) fp16(lB lBs), 16-byte aligned: the many-row path's LoRA B
   int8_t* q_out;             // (M, ld_q) int8 activations
   int ld_q;
   float* xs_out;             // (M) activation scale (an fp16 value)
@@ -174,7 +173,6 @@ struct SsmPrepArgs {
   const float* norm_w;       // (H P) fp32 gated-RMSNorm weight
   const int8_t* lB;          // (16, H P) LoRA B, int8 (null: no LoRA intermediate)
   const uint16_t* lBs;       // (16) fp16
-  const uint16_t* lBq;       // (16, K) fp16(lB lBs), 16-byte aligned: the many-row path's LoRA B
   int8_t* q_out;             // (M, ld_q) int8 activations
   int ld_q;
   float* xs_out;             // (M) activation scale (an fp16 value)
@@ -322,11 +320,8 @@ hipError_t launch_dequant_lora_b(const int8_t* B, const uint16_t* Bs, int K, uin
 hipError_t launch_proj(const ProjArgs& a, int M, int mode, hipStream_t s);
 hipError_t launch_prep(const PrepArgs& a, int M, int mode, hipStream_t s);
 hipError_t launch_gemm(const GemmArgs& a, int mode, hipStream_t s);
-// Prefill GEMM for thousands of rows (IN without conv, OUT): q in the wide tiled layout (rows
-// padded to 16); expands the bits to w8 (gemm_wide_w8_bytes of scratch, tiled likewise) and runs
-// a tiled MFMA GEMM with gemm_kernel's epilogue.
-size_t gemm_wide_w8_bytes(int N, int K);
-hipError_t launch_gemm_wide(const GemmArgs& a, int mode, int8_t* w8, hipStream_t s);
+// Prefill GEMM for many rows (IN without conv, OUT): q in the wide layout, with its row sums.
+hipError_t launch_gemm_wide(const GemmArgs& a, int mode, hipStream_t s);
 hipError_t launch_scaffold(const ScaffoldArgs& a, int M, hipStream_t s);
 hipError_t launch_scaffold_xchg(const ScaffoldArgs& a, int M, hipStream_t s);  // a.ws set, M <= 4
 hipError_t launch_tile_bits(const uint32_t* src, uint32_t* dst, int N, int KW, hipStream_t s);

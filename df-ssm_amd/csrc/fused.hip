@@ -354,17 +354,6 @@ __device__ __forceinline__ void norm_rows(FusedLds<M>& L, const PIn<M>& pi, cons
   }
 }
 
-// Within each quad of lanes (4i..4i+3, quad lane b = lane % 4): byte j of the result of lane b is
-// byte b of lane j's a (a 4 x 4 byte transpose: two DPP quad permutations and two byte selects).
-// v_perm_b32 (src0, src1, sel): byte k of the result is byte sel_k of the 8 bytes
-// {src1 bytes 0..3, src0 bytes 0..3}.
-__device__ __forceinline__ uint32_t quad_transpose_bytes(uint32_t a, int b) {
-  const uint32_t p = (uint32_t)dpp_i32<0x4E>((int)a);  // lane b ^ 2
-  const uint32_t u = __builtin_amdgcn_perm(p, a, (b & 2) ? 0x03020706u : 0x05040100u);
-  const uint32_t q = (uint32_t)dpp_i32<0xB1>((int)u);  // lane b ^ 1
-  return __builtin_amdgcn_perm(q, u, (b & 1) ? 0x03070105u : 0x06020400u);
-}
-
 // The int8 quantizer of the M rows (after norm_rows) on the data waves: the scale from the row's
 // amax, q into L.q in the GEMV's order, sum q into L.ri (0 from the other waves), the scale into
 // L.xs. One workgroup barrier; the caller passes another before the GEMV reads L.q.

@@ -208,8 +208,7 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& a, const GemmPro& p) {
   const int g = blockIdx.x;
   const int K = a.K, CH = K / 128;
   const int QS = K + 16;  // padded LDS row stride
-  // rows of this workgroup: blocks [blockIdx.y * bpw, +bpw) of the activation rows (one range
-  // in decode; the prompt prefill spreads its thousands of rows over gridDim.y ranges)
+  // rows of this workgroup: blocks [blockIdx.y * bpw, +bpw) of the activation rows
   // (PRO: the grid rows past p.gy hold the prologue workgroups, not row ranges)
   const int grows = PRO ? p.gy : (int)gridDim.y;
   const int nblk = (a.M + MP - 1) / MP, bpw = (nblk + grows - 1) / grows;
@@ -571,11 +570,10 @@ static hipError_t launch_gemm_mi(const GemmArgs& a, const GemmPro* pro, hipStrea
   // blocks pays each block's q-tile round trip and epilogue in turn: out_proj 7.0 -> 6.3 us at
   // batch 32, 18.5 -> 16.2 us at the 2.7B shape and batch 64); with 32 or 64 output rows per
   // workgroup (133..166 workgroups) the blocks stay in one workgroup (a second round measured
-  // slower). Many rows (prefill) are split into ranges so that the grid fills about two rounds.
+  // slower).
   const int gx = (a.N + 16 * RT - 1) / (16 * RT);
   const int nblk = (a.M + MI * 16 - 1) / (MI * 16);
-  int gy = a.M > 64 ? (512 + gx / 2) / gx : (RT == 1 ? nblk : 1);
-  gy = gy < 1 ? 1 : (gy > nblk ? nblk : gy);
+  const int gy = RT == 1 ? nblk : 1;
   int cus = 0;
   if (PRO) {
     int dev = 0;
@@ -634,167 +632,242 @@ static hipError_t launch_gemm_mode(const GemmArgs& a, const GemmPro* pro, hipStr
 }
 
 // ---------------------------------------------------------------------------------------------
-// Wide GEMM for the prompt prefill (thousands of activation rows). The sign bits are expanded once
-// per projection to int8 +-1 (expand_bits_kernel: W8 row-major (N, K)), then a plain MFMA GEMM:
-// a workgroup of 4 waves owns a 128 x 128 tile (activation rows x output rows), wave w the 64 x 64
-// quarter (rows 64 (w & 1), outputs 64 (w >> 1)) as 4 x 4 tiles of v_mfma_i32_16x16x64_i8, its A
-// (q) and B (W8) operands loaded straight into registers two k steps ahead (three-stage ring; loads
-// complete in issue order). Both operands are stored in 16-row tiles (wide_tiled_offset), so the
-// MFMA lane layout (lane l: row l % 16, 16 bytes of k block l / 16) is one contiguous 1 KiB per
-// wave-wide load; row-major rows K bytes apart put every lane on its own cache line. acc = sum_k q[m][k] W8[n][k] is exact (int32), i.e. gemm_kernel's
-// acc; the epilogue is gemm_kernel's, operation for operation (scales, LoRA term in fp64, proj
-// rows or residual add). Workgroup -> tile: workgroups are dealt to the 8 XCDs in turn, so XCD x
-// takes the row tiles m = x (mod 8) (each activation tile is read by one XCD's L2) and walks the
-// output tiles of one row tile after another.
+// Wide GEMM for the prompt prefill (more than 64 activation rows): a workgroup of 4 waves owns a
+// 64 x 64 TJ tile (activation rows x output rows), wave w all its rows and the 16 TJ outputs from
+// 16 TJ w, as TI x TJ tiles of v_mfma_i32_16x16x64_i8 (TI = 4).
+//
+// What bounds it is the path that feeds the matrix cores: a CU turns over 64 bytes of L1 and 128 of LDS
+// per clock, against 8192 operations. So the activations go through LDS once per workgroup (stages of
+// two k steps in three buffers: loaded two stages ahead, read up to one stage ahead), and the weights
+// stay sign bits up to the registers: a lane loads one 16-byte chunk of its output row per 512 columns
+// and makes each step's 0/1 bytes from it with two instructions per four (kWideTile: the layout of q);
+// the MFMA sums are then T = sum of q over the set bits, and the accumulator 2 T - sum q with the row
+// sums from the prologue. The next step's bytes and the next tiles' LDS reads are issued between the
+// MFMAs of the current one (sched_barrier keeps them there: a wave issues in order, and the four MFMAs
+// of a row tile leave the other pipes 60 clocks).
+//
+// The weights are the MFMA's A operand (result rows = outputs), row p of tile t being output
+// 4 TJ (p / 4) + 4 t + p % 4 of the wave: a lane (one activation row, result rows 4 g .. 4 g + 3) then
+// holds 4 TJ consecutive outputs over its TJ tiles, and the 64 outputs of a row leave as one 128-byte
+// line. The rank-16 LoRA term runs on the fp64 matrix cores as in gemm_kernel (its A rows permuted so
+// that the f64 result rows are the int8 ones), the rest of the epilogue is gemm_kernel's, operation for
+// operation. Three workgroups per CU (TJ = 4; five for TJ = 2), so that one's epilogue (the fp64
+// matrix instructions are 29% of the matrix time at K = 2560) runs beside the others' main loops.
+// Measured against a GEMM on weights expanded to bytes (4 waves of 64 x 64, both operands from L2
+// straight to registers, 16 fp64 fmas per element), with its expansion: in_proj of the 2.7B shape at
+// 16 384 rows 895 -> 404 us (2.2 POPS), out_proj 348 -> 166; of the 1.3B shape at 999 rows 67 -> 28 and
+// 43 -> 16 us. TI = 8 at TJ = 4 (two workgroups per CU): 381 and 169 us at 16 384 rows, 286 against
+// 278 for the 1.3B in_proj, 37 against 30 at 1000 rows.
+// Workgroup -> tile: workgroups are dealt to the 8 XCDs in turn; XCD x takes the x-th eighth of the
+// tiles in order, the output tiles of a row tile after another, so an activation tile is read by one
+// or two L2s and the weight bits stay in all of them.
 // ---------------------------------------------------------------------------------------------
-// W8 = bit k of row n ? +1 : -1 in the wide tiled layout; one thread per (row, 128-column chunk)
-// of the tiled bits.
-__global__ __launch_bounds__(256) void expand_bits_kernel(const uint32_t* __restrict__ bits, int8_t* __restrict__ w8,
-                                                          int N, int K) {
-  const int CH = K / 128;
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= N * CH) return;
-  const int n = i / CH, c = i - n * CH;
-  const u32x4 b = ld_nt(bits + (((size_t)(n >> 6) * CH + c) * 64 + (n & 63)) * 4);
-#pragma unroll
-  for (int q = 0; q < 8; ++q) {  // 16 columns 128 c + 16 q .. + 15: bits 16 q .. of the chunk
-    const uint32_t h16 = (b[q >> 1] >> (16 * (q & 1))) & 0xffffu;
-    uint32_t o[4];
-#pragma unroll
-    for (int nib = 0; nib < 4; ++nib) {
-      const uint32_t x = (((h16 >> (4 * nib)) & 0xfu) * 0x00204081u) & 0x01010101u;  // 0/1 bytes
-      o[nib] = __builtin_amdgcn_perm(0u, 0x000001ffu, x);                             // -> -1/+1
-    }
-    *(u32x4*)(w8 + wide_tiled_offset(n, 128 * c + 16 * q, K)) = u32x4{o[0], o[1], o[2], o[3]};
-  }
-}
-
-constexpr int kWT = 128;  // tile edge (rows and outputs)
-
-template <int MODE>
-__global__ __launch_bounds__(256) void gemm_wide_kernel(GemmArgs a, const int8_t* __restrict__ w8, int TN) {
-  __shared__ float hl[kWT][DFSSM_LORA_R];
-  __shared__ float xsl[kWT];
+template <int MODE, int TJ>
+__global__ __launch_bounds__(256, TJ == 4 ? 3 : 4) void gemm_wide_kernel(GemmArgs a, int TN, int tiles) {
+  constexpr int TI = 4;
+  constexpr int TM = 16 * TI, SB = TI * 2048;  // rows; bytes of a stage: [row tile][step][64 lanes][16]
+  constexpr int GL = TI / 2;                   // 16-byte vectors per thread and stage
+  constexpr int EX = 4 * TJ / TI;              // dwords of the next step's weights made per row tile
+  constexpr int RD = 3;                        // row tiles read ahead, in a ring of four
+  static_assert(2 * TI % 4 == 0 && EX * TI == 4 * TJ, "tile");
+  __shared__ __attribute__((aligned(16))) int8_t As[3 * SB];
+  __shared__ __attribute__((aligned(16))) float hl[TM][DFSSM_LORA_R];
+  __shared__ float xsl[TM];
+  __shared__ int qsl[TM];
+  const int per = (tiles + 7) / 8;
+  const int id = ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3);
+  if (((int)blockIdx.x >> 3) >= per || id >= tiles) return;  // uniform over the workgroup
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave & 1, wn = wave >> 1;
-  const int L = (int)blockIdx.x, xcd = L & 7, j = L >> 3;
-  const int tm = 8 * (j / TN) + xcd, tn = j % TN;
-  const int TM = (a.M + kWT - 1) / kWT;
-  if (tm >= TM) return;  // uniform over the workgroup
-  const int m0 = tm * kWT, n0 = tn * kWT, K = a.K, KS = K / 64;
-  const int lr = lane & 15;
-  // operand bases: 16-row tiles of the tiled layouts, lane l at byte 16 l of a (tile, k step)
-  // (tiles past the last one are clamped to it: their results are discarded)
-  const int lastA = (a.M + 15) / 16 - 1, lastB = (a.N + 15) / 16 - 1;
-  uint32_t ao[4], bo[4];
+  const int m0 = (id / TN) * TM, n0 = (id % TN) * (64 * TJ) + 16 * TJ * wave;
+  const int K = a.K, KS = K / 64, CH = K / 128, NS = KS / 2;
+  const int lr = lane & 15, g = lane >> 4;
+  // rows past the end re-read the last tile, outputs past it the last padded row; never stored
+  const int last_tile = (a.M + 15) / 16 - 1, last_n = (a.N + 63) / 64 * 64 - 1;
+  uint32_t ao[GL];
 #pragma unroll
-  for (int t = 0; t < 4; ++t) {
-    const int ta = (m0 + 64 * wm + 16 * t) >> 4, tb = (n0 + 64 * wn + 16 * t) >> 4;
-    ao[t] = (uint32_t)((ta < lastA ? ta : lastA) * KS * 1024 + 16 * lane);
-    bo[t] = (uint32_t)((tb < lastB ? tb : lastB) * KS * 1024 + 16 * lane);
+  for (int j = 0; j < GL; ++j) {
+    const int u = tid + 256 * j, t = (m0 >> 4) + (u >> 7);
+    ao[j] = (uint32_t)((t < last_tile ? t : last_tile) * KS * 1024 + (u & 127) * 16);
   }
-  v4i acc[4][4];
+  uint32_t bo[TJ];
 #pragma unroll
-  for (int ti = 0; ti < 4; ++ti)
+  for (int t = 0; t < TJ; ++t) {
+    int n = n0 + 4 * TJ * (lr >> 2) + 4 * t + (lr & 3);
+    n = n < last_n ? n : last_n;
+    bo[t] = (uint32_t)((((n >> 6) * CH + g) * 64 + (n & 63)) * 16);
+  }
+  u32x4 st[GL], wb[TJ], wn[TJ];
+  auto load_a = [&](int stage) {
+    const uint32_t o = 2048u * (uint32_t)(stage < NS ? stage : NS - 1);  // (past the end: unused)
 #pragma unroll
-    for (int tj = 0; tj < 4; ++tj) acc[ti][tj] = v4i{0, 0, 0, 0};
-  v4i A[3][4], B[3][4];
-  auto load = [&](int st, int step) {
-    const uint32_t ko = (uint32_t)(1024 * (step < KS ? step : KS - 1));  // the ring's overrun re-reads
-#pragma unroll
-    for (int t = 0; t < 4; ++t) A[st][t] = *(const v4i*)(a.q + ao[t] + ko);
-#pragma unroll
-    for (int t = 0; t < 4; ++t) B[st][t] = *(const v4i*)(w8 + bo[t] + ko);
+    for (int j = 0; j < GL; ++j) st[j] = *(const u32x4*)(a.q + (ao[j] + o));
   };
-  auto mma = [&](int st) {
+  auto stage_a = [&](int off) {
 #pragma unroll
-    for (int ti = 0; ti < 4; ++ti)
-#pragma unroll
-      for (int tj = 0; tj < 4; ++tj) acc[ti][tj] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[st][ti], B[st][tj], acc[ti][tj], 0, 0, 0);
+    for (int j = 0; j < GL; ++j) *(u32x4*)&As[off + (tid + 256 * j) * 16] = st[j];
   };
-  load(0, 0);
-  __builtin_amdgcn_sched_barrier(0);
-  load(1, 1);
-  __builtin_amdgcn_sched_barrier(0);
-  // whole groups of three steps (K / 64 = 8, 16, ... 80: the last group may run past KS; those
-  // steps multiply a re-read of step KS - 1 and are skipped)
-  for (int s = 0; s < KS; s += 3) {
-    load(2, s + 2);
-    __builtin_amdgcn_sched_barrier(0);
-    mma(0);
-    load(0, s + 3);
-    __builtin_amdgcn_sched_barrier(0);
-    if (s + 1 < KS) mma(1);
-    load(1, s + 4);
-    __builtin_amdgcn_sched_barrier(0);
-    if (s + 2 < KS) mma(2);
+  auto load_b = [&](u32x4 (&w)[TJ], int sb) {
+    const uint32_t o = 4096u * (uint32_t)(8 * sb < KS ? sb : KS / 8 - 1);
+#pragma unroll
+    for (int t = 0; t < TJ; ++t) w[t] = *(const u32x4*)((const uint8_t*)a.bits + (bo[t] + o));
+  };
+  load_a(0);
+  load_b(wb, 0);
+  // the tile's LoRA intermediates, scales and row sums
+  f32x4 hv[TI / 4];
+#pragma unroll
+  for (int j = 0; j < TI / 4; ++j) {
+    const int i = 4 * (tid + 256 * j), m = m0 + i / DFSSM_LORA_R;
+    hv[j] = *(const f32x4*)(a.h + (size_t)(m < a.M ? m : a.M - 1) * DFSSM_LORA_R + i % DFSSM_LORA_R);
+  }
+  const int mt = m0 + (tid & (TM - 1)) < a.M ? m0 + (tid & (TM - 1)) : a.M - 1;
+  const float xs_t = a.xs[mt];
+  const int qs_t = a.qsum[mt];
+  stage_a(0);
+  load_a(1);
+  v4i acc[TI][TJ];
+#pragma unroll
+  for (int i = 0; i < TI; ++i)
+#pragma unroll
+    for (int t = 0; t < TJ; ++t) acc[i][t] = v4i{0, 0, 0, 0};
+#pragma unroll
+  for (int j = 0; j < TI / 4; ++j) *(f32x4*)(&hl[0][0] + 4 * (tid + 256 * j)) = hv[j];
+  if (tid < TM) {
+    xsl[tid] = xs_t;
+    qsl[tid] = qs_t;
+  }
+  stage_a(SB);
+  lds_barrier();
+  v4i A[4], B[2][TJ];
+#pragma unroll
+  for (int r = 0; r < RD; ++r) A[r] = *(const v4i*)&As[(r % TI) * 2048 + (r / TI) * 1024 + 16 * lane];
+#pragma unroll
+  for (int t = 0; t < TJ; ++t)
+#pragma unroll
+    for (int d = 0; d < 4; ++d) B[0][t][d] = (int)(wb[t][d] & 0x01010101u);
+  int b0 = 0, b1 = SB, b2 = 2 * SB;  // buffers of this stage, the next and the one after
+  for (int sb = 0; sb < KS / 8; ++sb) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {  // the stages of a 512-column chunk
+      load_a(4 * sb + q + 2);
+      if (q == 0) load_b(wn, sb + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int hs = 0; hs < 2; ++hs) {
+        if (q == 3 && hs == 1) {  // the next step is the next chunk's first
+#pragma unroll
+          for (int t = 0; t < TJ; ++t) wb[t] = wn[t];
+        }
+#pragma unroll
+        for (int i = 0; i < TI; ++i) {
+          const int x = hs * TI + i, y = x + RD;  // row tile (step, tile) of the stage; the one to read
+          A[y & 3] = y < 2 * TI ? *(const v4i*)&As[b0 + (y % TI) * 2048 + (y / TI) * 1024 + 16 * lane]
+                                : *(const v4i*)&As[b1 + ((y - 2 * TI) % TI) * 2048 + 16 * lane];
+#pragma unroll
+          for (int t = 0; t < TJ; ++t)
+            acc[i][t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(B[hs][t], A[x & 3], acc[i][t], 0, 0, 0);
+#pragma unroll
+          for (int e = 0; e < EX; ++e) {
+            const int t = (i * EX + e) / 4, d = (i * EX + e) % 4;
+            B[hs ^ 1][t][d] = (int)((wb[t][d] >> ((2 * q + hs + 1) & 7)) & 0x01010101u);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      stage_a(b2);
+      lds_barrier();
+      const int b = b0;
+      b0 = b1;
+      b1 = b2;
+      b2 = b;
+    }
   }
 
-  // ---- epilogue (gemm_kernel's): the tile's LoRA intermediates and activation scales in LDS ----
-  for (int i = tid; i < kWT * DFSSM_LORA_R; i += 256) {
-    const int m = m0 + i / DFSSM_LORA_R;
-    (&hl[0][0])[i] = m < a.M ? a.h[(size_t)m * DFSSM_LORA_R + i % DFSSM_LORA_R] : 0.0f;
-  }
-  if (tid < kWT) xsl[tid] = m0 + tid < a.M ? a.xs[m0 + tid] : 0.0f;
-  __syncthreads();
-#pragma unroll  // (a runtime tj would index the accumulators dynamically: scratch memory)
-  for (int tj = 0; tj < 4; ++tj) {
-    const int n = n0 + 64 * wn + 16 * tj + lr;
-    if (n >= a.N) continue;
+  // ---- epilogue: lane = activation row 16 i + lr, outputs nl .. nl + 4 TJ - 1 ----
+  const int nl = n0 + 4 * TJ * g;
+  double aq[TJ][4];  // LoRA A (f64 A operand, row lr: result row 4 (lr % 4) + lr / 4), ranks 4 s + g
+  float ws[TJ][4];
+#pragma unroll
+  for (int t = 0; t < TJ; ++t) {
+    int n = n0 + 4 * TJ * (lr & 3) + 4 * t + (lr >> 2);
+    n = n < a.N ? n : a.N - 1;
     const u32x4 la = *(const u32x4*)(a.lA + (size_t)n * DFSSM_LORA_R);
-    const float as = h2f(a.lAs[n]), ws = h2f(a.wscale[n]);
-    double aqd[DFSSM_LORA_R];
+    const float as = h2f(a.lAs[n]);
 #pragma unroll
-    for (int rr = 0; rr < DFSSM_LORA_R; ++rr) aqd[rr] = (double)r16((float)(int8_t)(la[rr >> 2] >> (8 * (rr & 3))) * as);
-    uint16_t old[4][4];
-    if (MODE == DFSSM_MODE_OUT) {  // the residual rows, all loaded before any is used
+    for (int s = 0; s < 4; ++s) aq[t][s] = (double)r16((float)(int8_t)(la[s] >> (8 * g)) * as);
 #pragma unroll
-      for (int ti = 0; ti < 4; ++ti)
+    for (int e = 0; e < 4; ++e) ws[t][e] = h2f(a.wscale[nl + 4 * t + e < a.N ? nl + 4 * t + e : a.N - 1]);
+  }
+#pragma unroll
+  for (int i = 0; i < TI; ++i) {
+    const int m = m0 + 16 * i + lr;
+    uint16_t* op = a.out + (size_t)(m < a.M ? m : a.M - 1) * a.ld_out + nl;
+    u32x4 old[TJ / 2];  // (8 outputs; N is a multiple of 8)
+    if (MODE == DFSSM_MODE_OUT) {  // the residual row
+#pragma unroll
+      for (int u = 0; u < TJ / 2; ++u) old[u] = *(const u32x4*)(op + (nl + 8 * u < a.N ? 8 * u : -nl));
+    }
+    double hd[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) hd[s] = (double)hl[16 * i + lr][4 * s + g];
+    const float xs = xsl[16 * i + lr];
+    const int qs = qsl[16 * i + lr];
+#pragma unroll
+    for (int u = 0; u < TJ / 2; ++u) {
+      u32x4 o;
+#pragma unroll
+      for (int v = 0; v < 2; ++v) {
+        const int t = 2 * u + v;
+        v4d lo = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int s = 0; s < 4; ++s) lo = __builtin_amdgcn_mfma_f64_16x16x4f64(aq[t][s], hd[s], lo, 0, 0, 0);
+        uint32_t r[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const int m = m0 + 64 * wm + 16 * ti + 4 * (lane >> 4) + e;
-          old[ti][e] = a.out[(size_t)(m < a.M ? m : a.M - 1) * a.ld_out + n];
+          const int accv = 2 * acc[i][t][e] - qs;
+          const float y = r16(r16(r16((float)accv) * xs) * ws[t][e]);
+          const float out = r16((float)lo[e] + y);
+          const uint32_t ow = MODE == DFSSM_MODE_OUT ? old[u][2 * v + (e >> 1)] : 0u;
+          r[e] = MODE == DFSSM_MODE_IN ? f2h(out) : f2h(h2f((uint16_t)(ow >> (16 * (e & 1)))) + out);
         }
-    }
-#pragma unroll
-    for (int ti = 0; ti < 4; ++ti)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int mb = 64 * wm + 16 * ti + 4 * (lane >> 4) + e, m = m0 + mb;
-        if (m >= a.M) continue;
-        const int accv = acc[ti][tj][e];
-        const float y = r16(r16(r16((float)accv) * xsl[mb]) * ws);
-        double lo = 0.0;
-#pragma unroll
-        for (int rr = 0; rr < DFSSM_LORA_R; ++rr) lo += (double)hl[mb][rr] * aqd[rr];
-        const float out = r16((float)lo + y);
-        uint16_t* op = a.out + (size_t)m * a.ld_out + n;
-        if (MODE == DFSSM_MODE_IN) *op = f2h(out);
-        else *op = f2h(h2f(old[ti][e]) + out);
+        o[2 * v] = r[0] | (r[1] << 16);
+        o[2 * v + 1] = r[2] | (r[3] << 16);
       }
+      if (m < a.M && nl + 8 * u < a.N) *(u32x4*)(op + 8 * u) = o;
+    }
   }
 }
 
-size_t gemm_wide_w8_bytes(int N, int K) { return (size_t)(N + 15) / 16 * 16 * K; }
-
-hipError_t launch_gemm_wide(const GemmArgs& a, int mode, int8_t* w8, hipStream_t s) {
-  if (a.M < 1 || a.K % 512 || a.K > 5120 || !a.h || !a.xs || !a.lA || !a.lAs || !a.wscale || a.conv_state ||
-      a.acc_out || (mode != DFSSM_MODE_IN && mode != DFSSM_MODE_OUT))
-    return hipErrorInvalidValue;
-  const int CH = a.K / 128;
-  hipLaunchKernelGGL(expand_bits_kernel, dim3((a.N * CH + 255) / 256), dim3(256), 0, s, a.bits, w8, a.N, a.K);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  const int TM = (a.M + kWT - 1) / kWT, TN = (a.N + kWT - 1) / kWT;
-  const dim3 g(8 * ((TM + 7) / 8) * TN);
-  if (mode == DFSSM_MODE_IN) hipLaunchKernelGGL(gemm_wide_kernel<DFSSM_MODE_IN>, g, dim3(256), 0, s, a, w8, TN);
-  else hipLaunchKernelGGL(gemm_wide_kernel<DFSSM_MODE_OUT>, g, dim3(256), 0, s, a, w8, TN);
+template <int MODE, int TJ>
+static hipError_t launch_gemm_wide_tile(const GemmArgs& a, hipStream_t s) {
+  const int TN = (a.N + 64 * TJ - 1) / (64 * TJ), tiles = (a.M + 63) / 64 * TN;
+  hipLaunchKernelGGL((gemm_wide_kernel<MODE, TJ>), dim3((tiles + 7) / 8 * 8), dim3(256), 0, s, a, TN, tiles);
   return hipGetLastError();
 }
 
+// 256 outputs per workgroup when that leaves two workgroups per CU, else 128 (the narrow tile reads
+// every activation operand for half as many MFMAs, but splits finer): 1.3B out_proj at 1000 rows
+// (128 wide tiles) 20.9 -> 15.7 us, 2.7B in_proj at 512 rows (336) 25.0 -> 20.9; on the other side
+// 1.3B out_proj at 8192 rows (1024) 58.7 against 64.5, 2.7B in_proj at 1000 rows (672) 33.3 against 35.0.
+template <int MODE>
+static hipError_t launch_gemm_wide_mode(const GemmArgs& a, hipStream_t s) {
+  return (a.M + 63) / 64 * ((a.N + 255) / 256) >= 512 ? launch_gemm_wide_tile<MODE, 4>(a, s)
+                                                       : launch_gemm_wide_tile<MODE, 2>(a, s);
+}
+
+hipError_t launch_gemm_wide(const GemmArgs& a, int mode, hipStream_t s) {
+  if (a.M < 1 || a.M > kGemmMaxRows || a.K % 512 || a.K > 5120 || !a.h || !a.xs || !a.qsum || !a.lA || !a.lAs ||
+      !a.wscale || a.conv_state || a.acc_out || a.N % 8 || a.ld_out % 8 ||
+      ((uintptr_t)a.out & 15u))
+    return hipErrorInvalidValue;
+  if (mode == DFSSM_MODE_IN) return launch_gemm_wide_mode<DFSSM_MODE_IN>(a, s);
+  if (mode == DFSSM_MODE_OUT) return launch_gemm_wide_mode<DFSSM_MODE_OUT>(a, s);
+  return hipErrorInvalidValue;
+}
+
 hipError_t launch_gemm(const GemmArgs& a, int mode, hipStream_t s) {
-  if (a.M < 1 || a.M > kGemmMaxRows || a.K % 512 || a.K > 5120) return hipErrorInvalidValue;
+  if (a.M < 1 || a.M > 64 || a.K % 512 || a.K > 5120) return hipErrorInvalidValue;
   switch (mode) {
     case DFSSM_MODE_IN: return launch_gemm_mode<DFSSM_MODE_IN, false>(a, nullptr, s);
     case DFSSM_MODE_OUT: return launch_gemm_mode<DFSSM_MODE_OUT, false>(a, nullptr, s);

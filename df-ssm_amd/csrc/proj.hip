@@ -193,16 +193,16 @@ __global__ __launch_bounds__(kPT) void prep_kernel(PrepArgs a, int M) {
 }
 
 // ------------------------------------------------------------------------------------------
-// prep_rows_kernel<K / 512>: the same prologue for many rows (the prompt prefill runs thousands), one
+// prep_rows_kernel<K / 512>: the same prologue for many rows (prompt prefill, for the wide GEMM), one
 // workgroup of 16 waves per 16 rows. Wave w has row w in registers for the RMSNorm, the maximum and
 // the quantizer (no exchange between waves); the 16 x 16 LoRA intermediates of the workgroup are one
 // contraction over K and run on the fp64 matrix cores (v_mfma_f64_16x16x4f64: exact products of fp16
 // values, fp64 sums): the normalized rows go through LDS, up to 2560 columns at a time, each wave
 // takes 32 columns of every 512 and the waves' sums are added through LDS. Within an MFMA step lane
 // group g supplies column 8 g + s of a 32-column block for both operands (a permutation of k), so
-// both come as 16-byte vectors. With q_tiled the 16 rows of q are one contiguous block of the wide
-// GEMM's layout: staged in LDS (16-byte units, swizzled by their 16-column block: a row's units are 256
-// bytes apart) and stored as one. The decode-only outputs are not supported.
+// both come as 16-byte vectors. The 16 rows of q are one contiguous block of the wide GEMM's layout
+// (kWideTile): staged in LDS (the rows of the 16-byte units swizzled by step and group, which are
+// multiples of 256 bytes apart) and stored as one, the rows past M with copies of the last one.
 //
 // What bounds it: VALU issue (about 18 instructions per value) and the fp64 matrix rate, both about
 // 9 us per workgroup at K = 5120, one workgroup per CU. Measured against one workgroup of K / 8 threads
@@ -262,34 +262,35 @@ __global__ __launch_bounds__(kPrepRowsT) void prep_rows_kernel(PrepArgs a, int M
 #pragma unroll
   for (int j = 0; j < PC; ++j) bv[j] = *(const u32x4*)(lb + 512 * j);
   asm volatile("" ::: "memory");  // issued here, not sunk to their use
-  if (live && lane == 0 && a.xs_out) a.xs_out[m] = xs;
-  if (a.q_out) {
+  if (live && lane == 0) a.xs_out[m] = xs;
+  int qsum = 0;
 #pragma unroll
-    for (int j = 0; j < KB; ++j) {
-      uint32_t qw[2] = {0u, 0u};
+  for (int j = 0; j < KB; ++j) {
+    uint32_t qw[2] = {0u, 0u};
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int q = quant_i8(h2f((uint16_t)(v[j][e >> 1] >> (16 * (e & 1)))), rinv);
-        qw[e >> 2] |= (uint32_t)(q & 0xff) << (8 * (e & 3));
-      }
-      const uint2 qv = {qw[0], qw[1]};
-      if (a.q_tiled) {
-        const int blk = 32 * j + (lane >> 1);  // 16-column block; this lane's half of it
-        *(uint2*)&lds[256 * blk + 16 * (w ^ (blk & 15)) + 8 * (lane & 1)] = qv;
-      } else if (live) {
-        *(uint2*)(a.q_out + (size_t)m * a.ld_q + 512 * j + 8 * lane) = qv;
-      }
+    for (int e = 0; e < 8; ++e) {
+      const int q = quant_i8(h2f((uint16_t)(v[j][e >> 1] >> (16 * (e & 1)))), rinv);
+      qw[e >> 2] |= (uint32_t)(q & 0xff) << (8 * (e & 3));
     }
-    if (a.q_tiled) {
-      lds_barrier();
-      u32x4* qt = (u32x4*)(a.q_out + (size_t)m0 * K);  // the 16 rows of the tile
-      for (int u = tid; u < K; u += kPrepRowsT) {      // 16-byte units [blk][row]
-        const int blk = u >> 4, row = u & 15;
-        qt[u] = *(const u32x4*)&lds[256 * blk + 16 * (row ^ (blk & 15))];
-      }
-      lds_barrier();
+    // lane 16 gg + 4 d + b holds columns 128 gg + 32 d + 8 b + s (s = 0..7) of the chunk; after the
+    // transpose the four bytes b of s = b and of s = b + 4
+    const int b = lane & 3, d = (lane >> 2) & 3;
+    const int sw = w ^ (4 * b + g);  // swizzled row
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      qsum = __builtin_amdgcn_sdot4((int)qw[h], 0x01010101, qsum, false);
+      *(uint32_t*)&lds[((8 * j + b + 4 * h) * 64 + 16 * g + sw) * 16 + 4 * d] = quad_transpose_bytes(qw[h], b);
     }
   }
+  const int S = wave_sum_dpp_i32(qsum);
+  if (live && lane == 0) a.s_out[m] = S;
+  lds_barrier();
+  u32x4* qt = (u32x4*)(a.q_out + (size_t)m0 * K);  // the 16 rows of the tile
+  for (int u = tid; u < K; u += kPrepRowsT) {      // 16-byte units [step][g][row]
+    const int sw = (u & 15) ^ (4 * ((u >> 6) & 3) + ((u >> 4) & 3));
+    qt[u] = *(const u32x4*)&lds[((u & ~15) + sw) * 16];
+  }
+  lds_barrier();
   prep_v4d acc = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
   for (int j0 = 0; j0 < KB; j0 += PC) {
@@ -955,11 +956,10 @@ hipError_t launch_prep(const PrepArgs& a, int M, int mode, hipStream_t s) {
   if (mode == DFSSM_MODE_OUT && (!a.sumsq_slots || a.n_slots < 1 || a.n_slots > a.K / 8)) return hipErrorInvalidValue;
   if (a.lB && !a.lBs) return hipErrorInvalidValue;
   if (a.K > kMaxK || a.K % 512) return hipErrorInvalidValue;  // K / 8 threads: whole waves
-  // many rows: prep_rows_kernel
-  const bool rows_path = mode == DFSSM_MODE_IN && M > 64 && a.lBq && a.h_out && !a.planes_out && !a.xn_out &&
-                         !a.xs16_out && !a.s_out;
-  if (a.q_tiled && !rows_path) return hipErrorInvalidValue;
-  if (rows_path) {
+  if (a.q_tiled) {  // many rows
+    if (mode != DFSSM_MODE_IN || !a.lBq || !a.h_out || !a.q_out || !a.s_out || !a.xs_out || a.planes_out || a.xn_out ||
+        a.xs16_out)
+      return hipErrorInvalidValue;
     const dim3 g((M + 15) / 16);
     switch (a.K / 512) {
 #define DFSSM_PREP_KB(kb) \

@@ -107,10 +107,11 @@ def test_prefill_2p7b_layer_shapes():
     _prefill_vs_steps(w, 64, 20)
 
 
-@pytest.mark.parametrize("dm,di,B,T", [(1536, 3072, 5, 27), (1536, 3072, 7, 41), (512, 3584, 9, 29), (4608, 512, 6, 43)])
+@pytest.mark.parametrize("dm,di,B,T", [(1536, 3072, 5, 27), (1536, 3072, 5, 13), (512, 3584, 64, 19),
+                                        (4608, 512, 6, 43)])
 def test_prefill_many_rows(dm, di, B, T):
-    """The many-row prologue (more than 64 rows) at odd multiples of 512 columns, one and two passes of
-    the LoRA contraction, row counts no tile divides, q row-major (under 256 rows) and tiled."""
+    """The many-row prologue and GEMM (more than 64 rows) at odd multiples of 512 columns, one and two
+    passes of the LoRA contraction, row counts no tile divides, both widths of the GEMM's tile."""
     c = DFSSMConfig(n_layer=2, d_model=dm, d_inner=di, d_state=128, nheads=di // 64, headdim=64, ngroups=1,
                     vocab_size=1000, kw=4)
     print(f"prefill rows {B * T} of {dm} / {di}", flush=True)
