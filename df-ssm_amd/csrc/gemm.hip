@@ -846,13 +846,14 @@ static hipError_t launch_gemm_wide_tile(const GemmArgs& a, hipStream_t s) {
   return hipGetLastError();
 }
 
-// 256 outputs per workgroup when that leaves two workgroups per CU, else 128 (the narrow tile reads
+// 256 outputs per workgroup when that makes 640 workgroups (2.5 per CU), else 128 (the narrow tile reads
 // every activation operand for half as many MFMAs, but splits finer): 1.3B out_proj at 1000 rows
-// (128 wide tiles) 20.9 -> 15.7 us, 2.7B in_proj at 512 rows (336) 25.0 -> 20.9; on the other side
-// 1.3B out_proj at 8192 rows (1024) 58.7 against 64.5, 2.7B in_proj at 1000 rows (672) 33.3 against 35.0.
+// (128 wide tiles) 20.9 -> 15.7 us, 2.7B in_proj at 512 rows (336) 25.0 -> 20.9, 1.3B in_proj at 1000 rows
+// (544) 30.0 -> 27.8; on the other side 2.7B in_proj at 1000 rows (672) 33.3 against 35.0, 1.3B out_proj at
+// 8192 rows (1024) 58.7 against 64.5.
 template <int MODE>
 static hipError_t launch_gemm_wide_mode(const GemmArgs& a, hipStream_t s) {
-  return (a.M + 63) / 64 * ((a.N + 255) / 256) >= 512 ? launch_gemm_wide_tile<MODE, 4>(a, s)
+  return (a.M + 63) / 64 * ((a.N + 255) / 256) >= 640 ? launch_gemm_wide_tile<MODE, 4>(a, s)
                                                        : launch_gemm_wide_tile<MODE, 2>(a, s);
 }
 

@@ -14,6 +14,8 @@
 // together with the row-wise kernels the prefill equals, bit for bit, n calls of the decode step
 // (Mamba-2 recurrence of df_ssm_kernels.cu:53-103 / training/df_ssm_mamba2_distill_dfw.py:346-381,
 // evaluated token by token as the reference's cpu_inference_driver.py:186-204 ingests a prompt).
+#include <type_traits>
+
 #include "common.h"
 #include "dfssm_kernels.h"
 
@@ -130,9 +132,9 @@ __global__ __launch_bounds__(256) void conv_tokens_kernel(ConvTokArgs a) {
 //   tokens on full waves.
 // Measured per layer, against the map this replaces (ssm_kernel's own, two rows and four columns per
 // lane, whose reductions took two thirds of the instructions and which kept a head on one CU):
-// 4796 -> 1499 us at the 2.7B shape and 64 x 256 tokens (1.07 ms if the four instructions per
-// element issued back to back), 916 -> 187 us at the 1.3B shape and 1 x 999 tokens (W = 4), 32.6 ->
-// 9.4 us at 1 x 32.
+// 4796 -> 1483 us at the 2.7B shape and 64 x 256 tokens (1.07 ms if the four instructions per
+// element issued back to back; a wave-token takes 680 clocks of its SIMD for about 165 instructions),
+// 916 -> 150 us at the 1.3B shape and 1 x 999 tokens, 32.6 -> 8.4 us at 1 x 32 (W = 8).
 //
 // The readout's sum is ssm_kernel's tree: quads A_j of four columns summed in order from zero (the
 // product C h is exact in fp64, so an fma rounds as its multiply-then-add), Q_i = (A_4i + A_4i+1) +
@@ -141,14 +143,15 @@ __global__ __launch_bounds__(256) void conv_tokens_kernel(ConvTokArgs a) {
 // lanes apart, the waves:
 //   W = 1: group g holds Q_2g and Q_(2g ^ 3);
 //   W = 2: wave w holds Q_4w .. Q_4w+3, group g Q_4w + (-g mod 4);
-//   W = 4: wave w holds Q_2w (groups 0, 1: its halves) and Q_(2w ^ 3) (groups 2, 3).
+//   W = 4: wave w holds Q_2w (groups 0, 1: its halves) and Q_(2w ^ 3) (groups 2, 3);
+//   W = 8: wave w holds Q_w, group g its quad g.
 // More waves per block cost more instructions per element (the per-token work is shared by fewer
 // columns) and a partial sum through LDS, but fill the chip when there are few blocks
 // (launch_ssm_scan).
 //
 // Rounds of TT tokens are staged in LDS, double-buffered, their operands loaded one round ahead.
 // ------------------------------------------------------------------------------------------
-constexpr int scan_tt(int W) { return W == 1 ? 8 : 4 * W; }  // tokens per round
+constexpr int scan_tt(int W) { return W <= 2 ? 8 : 16; }  // tokens per round
 
 template <int W, int RB>
 struct ScanBuf {
@@ -166,9 +169,9 @@ struct ScanBuf {
 template <int W, int RB>
 struct ScanRaw {
   static constexpr int NT = 64 * W * RB, TT = scan_tt(W);
-  static constexpr int NI = TT * 16 * RB / NT;        // items per thread
+  static constexpr int NI = W == 1 ? TT / 4 : 1;      // items per thread (W = 8: of the first half)
   static constexpr int NB = TT * 32 / NT;             // 16-byte vectors of B | C per thread
-  static_assert(NI * NT == TT * 16 * RB && NB * NT == TT * 32, "whole vectors and items per thread");
+  static_assert(NB * NT == TT * 32 && (W == 8 ? 2 : 1) * TT * 16 * RB == NI * NT, "whole vectors and items");
   u32x4 bc[NB];
   uint16_t x[NI], z[NI];
   float dt[NI];
@@ -177,7 +180,7 @@ struct ScanRaw {
 
 template <int W, int RB>
 __device__ __forceinline__ int scan_item_token(int k) {
-  return W == 1 ? 4 * k + (((int)threadIdx.x & 63) >> 4) : (int)threadIdx.x / (16 * RB);
+  return W == 1 ? 4 * k + (((int)threadIdx.x & 63) >> 4) : (int)threadIdx.x / (16 * RB) % scan_tt(W);
 }
 template <int W, int RB>
 __device__ __forceinline__ int scan_item_row() {
@@ -237,8 +240,10 @@ __device__ __forceinline__ void scan_stage(ScanBuf<W, RB>& S, const ScanRaw<W, R
       for (int e = 0; e < 8; ++e) d[e] = (double)f[e];
     }
   }
+  if (W < 8 || tid < Raw::NT / 2) {
 #pragma unroll
-  for (int k = 0; k < Raw::NI; ++k) S.X[scan_item_token<W, RB>(k)][scan_item_row<W, RB>()] = h2f(r.x[k]) * r.dt[k];
+    for (int k = 0; k < Raw::NI; ++k) S.X[scan_item_token<W, RB>(k)][scan_item_row<W, RB>()] = h2f(r.x[k]) * r.dt[k];
+  }
   if (tid < Raw::TT) S.abar[tid] = r.abar;
 }
 
@@ -294,6 +299,35 @@ __device__ __forceinline__ void scan_quads(float* h, float abar, float X, float 
 #undef DFSSM_ROW
 }
 
+// One quad (W = 8): columns in lanes 0 and 1 of the row.
+__device__ __forceinline__ void scan_quad(float* h, float abar, float X, float b0, float b1, double c0, double c1, double& s0) {
+  float t0, t1, t2, t3;
+  double d0, d1, d2, d3;
+#define DFSSM_ROW(n) " row_newbcast:" n " row_mask:0xf bank_mask:0xf\n\t"
+  asm("v_mov_b64 %0, 0\n\t"
+      "s_nop 0\n\t"
+      "v_mul_f32_dpp %5, %15, %14" DFSSM_ROW("0")
+      "v_mul_f32_dpp %6, %16, %14" DFSSM_ROW("0")
+      "v_mul_f32_dpp %7, %15, %14" DFSSM_ROW("1")
+      "v_mul_f32_dpp %8, %16, %14" DFSSM_ROW("1")
+      "v_fma_f32 %1, %13, %1, %5\n\t"
+      "v_fma_f32 %2, %13, %2, %6\n\t"
+      "v_fma_f32 %3, %13, %3, %7\n\t"
+      "v_fma_f32 %4, %13, %4, %8\n\t"
+      "v_cvt_f64_f32 %9, %1\n\t"
+      "v_cvt_f64_f32 %10, %2\n\t"
+      "v_cvt_f64_f32 %11, %3\n\t"
+      "v_cvt_f64_f32 %12, %4\n\t"
+      "v_fmac_f64_dpp %0, %17, %9" DFSSM_ROW("0")
+      "v_fmac_f64_dpp %0, %18, %10" DFSSM_ROW("0")
+      "v_fmac_f64_dpp %0, %17, %11" DFSSM_ROW("1")
+      "v_fmac_f64_dpp %0, %18, %12" DFSSM_ROW("1")
+      : "=&v"(s0), "+v"(h[0]), "+v"(h[1]), "+v"(h[2]), "+v"(h[3]), "=&v"(t0), "=&v"(t1), "=&v"(t2), "=&v"(t3),
+        "=&v"(d0), "=&v"(d1), "=&v"(d2), "=&v"(d3)
+      : "v"(abar), "v"(X), "v"(b0), "v"(b1), "v"(c0), "v"(c1));
+#undef DFSSM_ROW
+}
+
 // The lane swaps on fp64 values: a's odd 16-lane rows change places with b's even ones; a's upper
 // 32 lanes with b's lower ones.
 __device__ __forceinline__ void swap16_f64(double& a, double& b) {
@@ -336,17 +370,17 @@ __global__ __launch_bounds__(64 * W * RB, 4) void ssm_scan_kernel(ScanArgs a) {
   const int rl = 16 * blk + r;
   const float Dh = a.D[head];
   // this lane's columns: quads 4 q .. of Qa and Qb, and its pair of columns for the broadcasts
-  const int Qa = W == 1 ? 2 * g : W == 2 ? 4 * w + ((4 - g) & 3) : (g < 2 ? 2 * w : (2 * w) ^ 3);
+  const int Qa = W == 1 ? 2 * g : W == 2 ? 4 * w + ((4 - g) & 3) : W == 4 ? (g < 2 ? 2 * w : (2 * w) ^ 3) : w;
   const int Qb = W == 1 ? Qa ^ 3 : Qa;
-  const int half = W == 4 ? 8 * (g & 1) : 0;
-  const int pair = W == 1 ? (r < 8 ? 8 * Qa + r : 8 * Qb + r - 8) : W == 2 ? 8 * Qa + (r & 7) : 8 * Qa + half / 2 + (r & 3);
+  const int part = W == 4 ? 8 * (g & 1) : W == 8 ? 4 * g : 0;  // first column within Qa
+  const int pair = W == 1 && r >= 8 ? 8 * Qb + r - 8 : 8 * Qa + part / 2 + (r & (W <= 2 ? 7 : W == 4 ? 3 : 1));
 
   Raw raw = scan_load<W, RB>(a, b, head, col0, 0);
   float* hp = a.h + (((size_t)b * a.H + head) * a.P + p0 + rl) * a.N;
   float h[4 * NQ];
 #pragma unroll
   for (int q = 0; q < NQ; ++q) {
-    const f32x4 v = ld_nt_f4(hp + 16 * (q < 4 ? Qa : Qb) + half + 4 * (q & 3));
+    const f32x4 v = ld_nt_f4(hp + 16 * (q < 4 ? Qa : Qb) + part + 4 * (q & 3));
     h[4 * q] = v.x; h[4 * q + 1] = v.y; h[4 * q + 2] = v.z; h[4 * q + 3] = v.w;
   }
   scan_stage<W, RB>(buf[0], raw);
@@ -372,28 +406,51 @@ __global__ __launch_bounds__(64 * W * RB, 4) void ssm_scan_kernel(ScanArgs a) {
     for (int k = 0; k < TT / 4; ++k) {
       if (4 * k >= nt) break;
       double acc[4];
+      auto tokens = [&](auto full_t) {  // FULL: all four tokens exist (all but a prompt's last ones)
+        constexpr bool FULL = decltype(full_t)::value;
+        // W > 1: few waves per SIMD, so the four tokens' operands are read before the first is used
+        constexpr int PF = W > 1 && FULL ? 4 : 1;
+        float2 bp[PF];
+        double c0[PF], c1[PF];
+        float X[PF], abar[PF];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int t = 4 * k + j;
-        acc[j] = 0.0;
-        if (t >= nt) continue;  // uniform: past the prompt's end
-        const float2 bp = *(const float2*)&S.bf[t][2 * pair];
-        const double c0 = S.cd[t][2 * pair], c1 = S.cd[t][2 * pair + 1];
-        const float X = S.X[t][rl], abar = S.abar[t];
-        double A[8 / W];
-        scan_quads<0>(h, abar, X, bp.x, bp.y, c0, c1, A[0], A[1]);
-        double q = A[0] + A[1];
-        if constexpr (NQ > 2) {
-          scan_quads<1>(h + 8, abar, X, bp.x, bp.y, c0, c1, A[2], A[3]);
-          q = q + (A[2] + A[3]);
+        for (int j = 0; j < 4; ++j) {
+          if (j % PF == 0) {
+#pragma unroll
+            for (int u = 0; u < PF; ++u) {
+              const int t = 4 * k + j + u;
+              bp[u] = *(const float2*)&S.bf[t][2 * pair];
+              c0[u] = S.cd[t][2 * pair];
+              c1[u] = S.cd[t][2 * pair + 1];
+              X[u] = S.X[t][rl];
+              abar[u] = S.abar[t];
+            }
+            if (PF > 1) __builtin_amdgcn_sched_barrier(0);
+          }
+          acc[j] = 0.0;
+          if (!FULL && 4 * k + j >= nt) continue;  // uniform: past the prompt's end
+          const int u = j % PF;
+          double A[NQ], q;
+          if constexpr (NQ == 1) {
+            scan_quad(h, abar[u], X[u], bp[u].x, bp[u].y, c0[u], c1[u], q);
+          } else {
+            scan_quads<0>(h, abar[u], X[u], bp[u].x, bp[u].y, c0[u], c1[u], A[0], A[1]);
+            q = A[0] + A[1];
+          }
+          if constexpr (NQ > 2) {
+            scan_quads<1>(h + 8, abar[u], X[u], bp[u].x, bp[u].y, c0[u], c1[u], A[2], A[3]);
+            q = q + (A[2] + A[3]);
+          }
+          if constexpr (NQ > 4) {
+            scan_quads<2>(h + 16, abar[u], X[u], bp[u].x, bp[u].y, c0[u], c1[u], A[4], A[5]);
+            scan_quads<3>(h + 24, abar[u], X[u], bp[u].x, bp[u].y, c0[u], c1[u], A[6], A[7]);
+            q = q + ((A[4] + A[5]) + (A[6] + A[7]));
+          }
+          acc[j] = q;
         }
-        if constexpr (NQ > 4) {
-          scan_quads<2>(h + 16, abar, X, bp.x, bp.y, c0, c1, A[4], A[5]);
-          scan_quads<3>(h + 24, abar, X, bp.x, bp.y, c0, c1, A[6], A[7]);
-          q = q + ((A[4] + A[5]) + (A[6] + A[7]));
-        }
-        acc[j] = q;
-      }
+      };
+      if (W > 1 && 4 * k + 4 <= nt) tokens(std::true_type{});
+      else tokens(std::false_type{});
       const double s = reduce4(acc[0], acc[1], acc[2], acc[3]);
       if constexpr (W == 1) finish(s, k);
       else S.part[w][4 * k + g][rl] = s;
@@ -403,14 +460,19 @@ __global__ __launch_bounds__(64 * W * RB, 4) void ssm_scan_kernel(ScanArgs a) {
     if constexpr (W > 1) {
       // (the partials of a buffer are rewritten two rounds later, after the next round's barrier)
       const int t = scan_item_token<W, RB>(0), i = scan_item_row<W, RB>();
-      double s = S.part[0][t][i] + S.part[1][t][i];
+      double s;
+      if constexpr (W == 8)
+        s = ((S.part[0][t][i] + S.part[3][t][i]) + (S.part[2][t][i] + S.part[1][t][i])) +
+            ((S.part[4][t][i] + S.part[7][t][i]) + (S.part[6][t][i] + S.part[5][t][i]));
+      else
+        s = S.part[0][t][i] + S.part[1][t][i];
       if constexpr (W == 4) s = s + (S.part[2][t][i] + S.part[3][t][i]);
-      finish(s, 0);
+      if (W < 8 || tid < Raw::NT / 2) finish(s, 0);
     }
   }
 #pragma unroll
   for (int q = 0; q < NQ; ++q)
-    st_nt_f4(hp + 16 * (q < 4 ? Qa : Qb) + half + 4 * (q & 3), f32x4{h[4 * q], h[4 * q + 1], h[4 * q + 2], h[4 * q + 3]});
+    st_nt_f4(hp + 16 * (q < 4 ? Qa : Qb) + part + 4 * (q & 3), f32x4{h[4 * q], h[4 * q + 1], h[4 * q + 2], h[4 * q + 3]});
 }
 
 // dst[b] = src[b * T + T - 1]: the last token's row of every sequence.
@@ -436,16 +498,21 @@ hipError_t launch_conv_tokens(const ConvTokArgs& args, int batch, hipStream_t s)
 
 hipError_t launch_ssm_scan(const ScanArgs& a, int batch, hipStream_t s) {
   if (a.T < 1 || a.P % 16 || a.N != 128) return hipErrorInvalidValue;
-  // Waves per 16-row block: the fewest that leave two waves per SIMD (2048 on the chip), where the
-  // head has enough blocks for a workgroup of four waves
+  // Waves per 16-row block: one where the head has the blocks for a workgroup of four waves and there
+  // are enough of them, more where the chip would be idle. Microseconds per 128 tokens with 1 / 2 / 4 / 8
+  // waves at the 1.3B shape (256 blocks per sequence): 1 sequence 59 / 35 / 24.6 / 22.4, 2: 60 / 36.7 /
+  // 36.0 / 42.3, 4: 63 / 53 / 63 / 79, 12: 134 / 129 / 170 / 227, 16: 170 / 166 / 224 / 303, 64: 589 / 608 /
+  // 876 / 1213.
   const int blocks = a.P / 16;
-  const long long waves = (long long)batch * a.H * blocks;
-  if (blocks % 4 == 0 && waves >= 2048)
+  const long long n = (long long)batch * a.H * blocks;
+  if (blocks % 4 == 0 && n >= 4096)
     hipLaunchKernelGGL((ssm_scan_kernel<1, 4>), dim3(a.H * (blocks / 4), batch), dim3(256), 0, s, a);
-  else if (blocks % 2 == 0 && 2 * waves >= 2048)
+  else if (blocks % 2 == 0 && n >= 1024)
     hipLaunchKernelGGL((ssm_scan_kernel<2, 2>), dim3(a.H * (blocks / 2), batch), dim3(256), 0, s, a);
-  else
+  else if (n > 256)
     hipLaunchKernelGGL((ssm_scan_kernel<4, 1>), dim3(a.H * blocks, batch), dim3(256), 0, s, a);
+  else
+    hipLaunchKernelGGL((ssm_scan_kernel<8, 1>), dim3(a.H * blocks, batch), dim3(512), 0, s, a);
   return hipGetLastError();
 }
 

@@ -126,20 +126,22 @@ def test_prefill_rejects_bad_prompts(tiny_weights):
         gpu.prefill(torch.full((2, 4), tiny_weights.cfg.vocab_size, dtype=torch.int64))
 
 
-@pytest.mark.parametrize("B,T,heads,headdim", [(5, 18, 16, 64), (5, 4, 16, 64), (17, 9, 16, 64), (24, 7, 32, 32),
-                                               (32, 13, 16, 64), (40, 1, 16, 64), (64, 5, 64, 16)])
+@pytest.mark.parametrize("B,T,heads,headdim", [(5, 18, 8, 64), (8, 37, 32, 16), (5, 21, 16, 64), (64, 6, 32, 16),
+                                               (5, 4, 16, 64), (17, 9, 16, 64), (24, 7, 32, 32), (64, 13, 16, 64),
+                                               (64, 1, 16, 64)])
 def test_prefill_readout_order(B, T, heads, headdim):
-    """The scan's C.h sums are added in the order of the batched decode step, in each of its forms (four,
-    two and one waves per 16-row block: B * 1024 / 16 blocks on a chip of 1024 SIMDs). A state of large
+    """The scan's C.h sums are added in the order of the batched decode step, in each of its forms (eight,
+    four, two and one waves per 16-row block: up to 256 blocks, under 1024, under 4096, more). A state of large
     values that cancel in pairs (C constant, B zero) makes every fp64 sum depend on its order, by far
     more than the fp16 rounding of y."""
-    c = DFSSMConfig(n_layer=1, d_model=512, d_inner=1024, d_state=128, nheads=heads, headdim=headdim, ngroups=1,
+    di = heads * headdim
+    c = DFSSMConfig(n_layer=1, d_model=512, d_inner=di, d_state=128, nheads=heads, headdim=headdim, ngroups=1,
                     vocab_size=1000, kw=4)
     w = make_weights(c, seed=3)
     L = w.layers[0]
-    L["conv_w"][1024:] = 0
-    L["conv_b"][1024:1152] = 0          # B = silu(0) = 0
-    L["conv_b"][1152:] = 1.5            # C = one constant
+    L["conv_w"][di:] = 0
+    L["conv_b"][di:di + 128] = 0        # B = silu(0) = 0
+    L["conv_b"][di + 128:] = 1.5        # C = one constant
     rng = np.random.default_rng(4)
     P = headdim
     big = (rng.uniform(1, 2, (B, heads, P, 32)) * 2.0 ** 50).astype(np.float32)
