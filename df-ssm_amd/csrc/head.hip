@@ -867,20 +867,29 @@ static hipError_t launch_head_i8s(const HeadArgs& a, int M, hipStream_t s) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// Batched head (M = 5..64): logits on the fp16 matrix cores, v_mfma_f32_16x16x32_f16. A = xf
-// (fp16, 16 rows x 32 k), B = 16 vocabulary rows of the int8 table converted exactly to fp16 in
-// registers. Products are exact; the sum is accumulated in fp32 (not exact -- the 1..4-row kernel
-// above is). One workgroup (4 waves) owns 256 vocabulary rows (each wave 4 tiles of 16); xf is
-// staged in LDS 512 columns at a time. Argmax as above: per-workgroup pairs, then the last
-// workgroup to finish reduces them.
+// Batched head on an fp16 table (M = 5..64): logits on the fp16 matrix cores,
+// v_mfma_f32_16x16x32_f16. A = xf (fp16, 16 rows x 32 k), B = 16 vocabulary rows. Products are exact;
+// the sum is accumulated in fp32 in k order (not exact -- the 1..4-row kernel above is).
+//
+// Bound by the stream of the table (206 MB at the 1.3B shape, 257 MB at the 2.7B), so the point is
+// bytes in flight: a workgroup of 16 waves owns 256 vocabulary rows (one per CU), each wave 16 of
+// them with eight k steps (8 KiB) on their way in a register ring, 128 KiB per CU, and nothing in the
+// loop waits for more than the oldest step. xf goes through LDS 512 columns at a time, double-buffered,
+// the next chunk loaded under the current one. Measured at the 2.7B shape and 64 rows against 4 waves
+// of 64 vocabulary rows with two steps in flight and xf staged behind two full barriers per chunk:
+// 233 -> 111 us in the decode step (where the state stream's dirty lines leave the last-level cache
+// under it), 85 us back to back (3.1 TB/s; 58 us at 5 rows, 4.4 TB/s). 4 or 16 steps in flight measure
+// the same, temporal loads 92 us.
+// Argmax as above: per-workgroup pairs, then the last workgroup to finish reduces them.
 // ---------------------------------------------------------------------------------------------
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4m __attribute__((ext_vector_type(4)));
 
-constexpr int kHT = 256;
-constexpr int kHV = 256;   // vocabulary rows per workgroup
+constexpr int kHT = 1024;
+constexpr int kHV = 256;   // vocabulary rows per workgroup (16 per wave)
 constexpr int kHK = 512;   // k chunk
 constexpr int kHS = kHK + 8;  // LDS row stride of the xf tile (halves)
+constexpr int kHR = 8;        // table steps in flight per wave
 
 // xf[m] = fp16((x * r) * norm_f) for the batched head (one workgroup per row).
 __global__ __launch_bounds__(256) void final_norm_kernel(const uint16_t* __restrict__ x, const float* __restrict__ norm_f,
@@ -896,100 +905,78 @@ __global__ __launch_bounds__(256) void final_norm_kernel(const uint16_t* __restr
   for (int k = tid; k < D; k += 256) xf[(size_t)m * D + k] = f2h((h2f(xm[k]) * r) * norm_f[k]);
 }
 
-template <int MI, bool F16>
+template <int MI>
 __global__ __launch_bounds__(kHT) void head_mfma_kernel(HeadArgs a, int M) {
   constexpr int MP = MI * 16;
-  __shared__ __attribute__((aligned(16))) uint16_t xs[MP][kHS];
-  __shared__ float wbest[4][MP];
-  __shared__ int widx[4][MP];
+  __shared__ __attribute__((aligned(16))) uint16_t xs[2][MP][kHS];
+  __shared__ float wbest[16][MP];
+  __shared__ int widx[16][MP];
   __shared__ bool is_last;
   __shared__ int next_tok[MP];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int D = a.D, CH = F16 ? D / 8 : D / 16;
-  const int v0 = blockIdx.x * kHV + wave * 64;
-  const int vpad = (a.V + 63) / 64 * 64;
-
-  f32x4m acc[4][MI];
+  const int lr = lane & 15, g = lane >> 4;
+  const int D = a.D, CH = D / 8, NC = D / kHK;
+  const int v = blockIdx.x * kHV + wave * 16 + lr;  // this lane's vocabulary row
+  // the tiled table holds V rounded up to 64 rows; rows past it re-read the last one (never stored)
+  const int vpad = (a.V + 63) / 64 * 64, vc = v < vpad ? v : vpad - 1;
+  const uint8_t* tab = a.emb + (((size_t)(vc >> 6) * CH + g) * 64 + (vc & 63)) * 16;  // step ks: + 4096 ks
+  u32x4 ring[kHR], st[MI];
 #pragma unroll
-  for (int vt = 0; vt < 4; ++vt)
+  for (int i = 0; i < kHR; ++i) ring[i] = ld_nt(tab + (size_t)4096 * i);
+  // xf chunk c: thread tid's vectors tid + 1024 i of the MP x 64 (rows past M re-read row M - 1)
+  auto load_xf = [&](int c) {
 #pragma unroll
-    for (int ib = 0; ib < MI; ++ib) acc[vt][ib] = f32x4m{0.f, 0.f, 0.f, 0.f};
-
-  for (int t = 0; t < D / kHK; ++t) {
-    __syncthreads();
-    for (int i = tid; i < MP * (kHK / 8); i += kHT) {  // 16-byte vectors of the xf chunk
-      const int row = i / (kHK / 8), c8 = i % (kHK / 8);
-      u32x4 v = {0u, 0u, 0u, 0u};
-      if (row < M) v = *(const u32x4*)(a.xf + (size_t)row * D + t * kHK + c8 * 8);
-      *(u32x4*)&xs[row][c8 * 8] = v;
+    for (int i = 0; i < MI; ++i) {
+      const int row = (tid >> 6) + 16 * i;
+      st[i] = *(const u32x4*)(a.xf + (size_t)(row < M ? row : M - 1) * D + (c < NC ? c : NC - 1) * kHK + (tid & 63) * 8);
     }
-    __syncthreads();
-#pragma unroll 2
+  };
+  auto stage_xf = [&](int b) {
+#pragma unroll
+    for (int i = 0; i < MI; ++i) *(u32x4*)&xs[b][(tid >> 6) + 16 * i][(tid & 63) * 8] = st[i];
+  };
+  load_xf(0);
+  f32x4m acc[MI];
+#pragma unroll
+  for (int ib = 0; ib < MI; ++ib) acc[ib] = f32x4m{0.f, 0.f, 0.f, 0.f};
+  stage_xf(0);
+  lds_barrier();
+  const int last = NC * (kHK / 32) - 1;  // last step: the ring's overrun re-reads it
+  for (int c = 0; c < NC; ++c) {
+    load_xf(c + 1);
+    __builtin_amdgcn_sched_barrier(0);  // issued here, not sunk to their stores
+#pragma unroll
     for (int ks = 0; ks < kHK / 32; ++ks) {
-      const int kl = ks * 32 + 8 * (lane >> 4);
-      const int k = t * kHK + kl;
+      const int kl = ks * 32 + 8 * g;
+      const f16x8 B = __builtin_bit_cast(f16x8, ring[ks % kHR]);
       f16x8 A[MI];
 #pragma unroll
-      for (int ib = 0; ib < MI; ++ib) A[ib] = *(const f16x8*)&xs[ib * 16 + (lane & 15)][kl];
+      for (int ib = 0; ib < MI; ++ib) A[ib] = *(const f16x8*)&xs[c & 1][ib * 16 + lr][kl];
 #pragma unroll
-      for (int vt = 0; vt < 4; ++vt) {
-        const int v = v0 + vt * 16 + (lane & 15);
-        // the tiled table holds V rounded up to 64 rows (zero padded); the last tile may pass it
-        f16x8 B;
-        if (F16) {
-          const u32x4 e16 = v < vpad ? *(const u32x4*)(a.emb + (((size_t)(v >> 6) * CH + (k >> 3)) * 64 + (v & 63)) * 16)
-                                     : u32x4{0u, 0u, 0u, 0u};
-          B = __builtin_bit_cast(f16x8, e16);
-        } else {
-          const uint2 e8 = v < vpad ? *(const uint2*)(a.emb + (((size_t)(v >> 6) * CH + (k >> 4)) * 64 + (v & 63)) * 16 + (k & 15))
-                                    : make_uint2(0u, 0u);
-#pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            const uint32_t w = e < 4 ? e8.x : e8.y;
-            B[e] = (_Float16)(float)(int8_t)(w >> (8 * (e & 3)));
-          }
-        }
-#pragma unroll
-        for (int ib = 0; ib < MI; ++ib) acc[vt][ib] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[ib], B, acc[vt][ib], 0, 0, 0);
-      }
+      for (int ib = 0; ib < MI; ++ib) acc[ib] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[ib], B, acc[ib], 0, 0, 0);
+      const int nx = c * (kHK / 32) + ks + kHR;
+      ring[ks % kHR] = ld_nt(tab + (size_t)4096 * (nx < last ? nx : last));
+      __builtin_amdgcn_sched_barrier(0);
     }
+    stage_xf((c + 1) & 1);  // (read by everyone before the last barrier)
+    lds_barrier();
   }
 
-  // logits and per-row best of this wave: element (vt, ib, j) is row m = 16 ib + 4 (lane/16) + j,
-  // vocabulary v = v0 + 16 vt + lane % 16
-  float best[MI][4];
-  int bidx[MI][4];
-#pragma unroll
-  for (int ib = 0; ib < MI; ++ib)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) { best[ib][j] = -INFINITY; bidx[ib][j] = 0x7fffffff; }
-#pragma unroll
-  for (int vt = 0; vt < 4; ++vt) {
-    const int v = v0 + vt * 16 + (lane & 15);
-    if (v >= a.V) continue;
-    const float sc = F16 ? 1.0f : h2f(a.emb_scale[v]);
-#pragma unroll
-    for (int ib = 0; ib < MI; ++ib)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int m = ib * 16 + 4 * (lane >> 4) + j;
-        if (m >= M) continue;
-        const uint16_t lh = F16 ? f2h(acc[vt][ib][j]) : f2h(acc[vt][ib][j] * sc);
-        if (a.logits) a.logits[(size_t)m * a.V + v] = lh;
-        const float lv = h2f(lh);
-        if (lv > best[ib][j]) { best[ib][j] = lv; bidx[ib][j] = v; }  // v increases with vt
-      }
-  }
-  // reduce over the 16 lanes that share (lane / 16), then over the 4 waves
+  // logits and per-row best of this wave: element (ib, j) is row m = 16 ib + 4 (lane / 16) + j,
+  // vocabulary row v
 #pragma unroll
   for (int ib = 0; ib < MI; ++ib)
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      float b = best[ib][j];
-      int bi = bidx[ib][j];
+      const int m = ib * 16 + 4 * g + j;
+      const uint16_t lh = f2h(acc[ib][j]);
+      if (v < a.V && m < M && a.logits) a.logits[(size_t)m * a.V + v] = lh;
+      float b = -INFINITY;
+      int bi = 0x7fffffff;
+      const float lv = h2f(lh);
+      if (v < a.V && lv > b) { b = lv; bi = v; }
       row_argmax_dpp(b, bi);  // the 16 lanes of the row group
-      if ((lane & 15) == 0) {
-        const int m = ib * 16 + 4 * (lane >> 4) + j;
+      if (lr == 0) {
         wbest[wave][m] = b;
         widx[wave][m] = bi;
       }
@@ -999,11 +986,7 @@ __global__ __launch_bounds__(kHT) void head_mfma_kernel(HeadArgs a, int M) {
     float b = wbest[0][tid];
     int bi = widx[0][tid];
 #pragma unroll
-    for (int w = 1; w < 4; ++w) {
-      const float ob = wbest[w][tid];
-      const int oi = widx[w][tid];
-      if (ob > b || (ob == b && oi < bi)) { b = ob; bi = oi; }
-    }
+    for (int w = 1; w < 16; ++w) argmax_take(b, bi, wbest[w][tid], widx[w][tid]);
     a.part_val[(size_t)tid * gridDim.x + blockIdx.x] = b;
     a.part_idx[(size_t)tid * gridDim.x + blockIdx.x] = bi;
   }
@@ -1016,11 +999,10 @@ __global__ __launch_bounds__(kHT) void head_mfma_kernel(HeadArgs a, int M) {
   __syncthreads();
   if (!is_last) return;
   __threadfence();
-  for (int r0 = 0; r0 < MI * 4; r0 += 4)  // four rows per wave at a time (registers)
-    argmax_pairs<4, 4, kHeadMaxGroups / 256>(a, M, (int)gridDim.x, next_tok, r0);
+  argmax_pairs<16, MI, kHeadMaxGroups / 256>(a, M, (int)gridDim.x, next_tok);
   if (tid == 0) *a.ticket = 0u;
   __syncthreads();
-  if (a.x_next) embed_next<F16, kHT>(a, next_tok, M, D);
+  if (a.x_next) embed_next<true, kHT>(a, next_tok, M, D);
 }
 
 hipError_t launch_head_batched(const HeadArgs& a, int M, hipStream_t s) {
@@ -1044,11 +1026,8 @@ hipError_t launch_head_batched(const HeadArgs& a, int M, hipStream_t s) {
   if (e != hipSuccess) return e;
   const int groups = (a.V + kHV - 1) / kHV;
   const int mi = (M + 15) / 16;
-#define DFSSM_HEAD_MFMA(MI)                                                                        \
-  if (mi == MI) {                                                                                 \
-    if (a.f16) hipLaunchKernelGGL((head_mfma_kernel<MI, true>), dim3(groups), dim3(kHT), 0, s, a, M); \
-    else hipLaunchKernelGGL((head_mfma_kernel<MI, false>), dim3(groups), dim3(kHT), 0, s, a, M);      \
-  }
+#define DFSSM_HEAD_MFMA(MI) \
+  if (mi == MI) hipLaunchKernelGGL((head_mfma_kernel<MI>), dim3(groups), dim3(kHT), 0, s, a, M);
   DFSSM_HEAD_MFMA(1)
   DFSSM_HEAD_MFMA(2)
   DFSSM_HEAD_MFMA(3)

@@ -418,3 +418,31 @@ def test_2p7b_layer_shapes_batch64():
     lo, _ = orc.step(ref[:, -1])
     assert np.abs(lg - lo.astype(np.float32)).max() == 0.0
     assert gpu.error_flag() == 0
+
+
+@pytest.mark.parametrize("B,vocab", [(5, 1000), (16, 257), (17, 4096), (33, 1025), (48, 64), (64, 50288)])
+def test_fp16_table_head_rows(B, vocab):
+    """The batched fp16-table head at the edges of its tiles (16-row blocks of sequences, 256-row
+    workgroups of the table, vocabularies no tile divides): logits against fp64 sums of the same fp16
+    values. Each is a sum of D = 1024 exact products in fp32 (error at most D 2^-24 sum |x e|, far below
+    the fp16 rounding that follows unless the sum cancels) rounded to fp16 (2^-11)."""
+    from dfssm import _C
+    from dfssm.format import DFSSMConfig
+    c = DFSSMConfig(n_layer=1, d_model=1024, d_inner=1024, d_state=128, nheads=16, headdim=64, ngroups=1,
+                    vocab_size=vocab, kw=4, emb_code=0)
+    w = make_weights(c, seed=9)
+    m = DFSSMModel.from_weights(w, device=DEV, batch_size=B)
+    print(f"fp16 head B={B} V={vocab}", flush=True)
+    g = torch.Generator().manual_seed(B)
+    m.x.copy_((2 * torch.randn(B, c.d_model, generator=g)).half())
+    _C.check(_C.lib().dfssm_lmhead_argmax(m._model, m.x.data_ptr(), m.workspace.data_ptr(), m.logits.data_ptr(),
+                                          m._next.data_ptr(), None, _C.stream()), "lmhead")
+    x = m.x.cpu().float()
+    r = 1.0 / torch.sqrt((x.double() ** 2).sum(1).float() * (1.0 / c.d_model) + 1e-5)
+    xf = ((x * r[:, None]) * torch.from_numpy(w.norm_f.astype(np.float32))).half().double()
+    e = torch.from_numpy(w.emb).double()
+    ref, mag = xf @ e.t(), xf.abs() @ e.abs().t()
+    got = m.logits.cpu().double()
+    assert ((got - ref).abs() <= ref.abs() * 2.0 ** -11 + 2.0 ** -24 + mag * c.d_model * 2.0 ** -24).all()
+    np.testing.assert_array_equal(m._next.cpu().numpy(), _np16(m.logits).astype(np.float32).argmax(axis=1))
+    assert m.error_flag() == 0
