@@ -104,9 +104,11 @@ __device__ __forceinline__ float dev_log1pf(float y) {  // y >= 0
 // (butterflies within 4 lanes), row_ror:4 = 0x124 and row_ror:8 = 0x128 (rotations within a row
 // of 16 lanes). After the four steps every lane holds its row's total; the four row totals are
 // then read from lanes 0, 16, 32, 48, so the result is uniform and the summation order is the
-// same in every wave.
+// same in every wave. (bound_ctrl, so that no old value takes part: with an explicit old value of zero
+// every step cost a move of it, 240 instructions of the one-launch layer; none of these controls reads
+// past its row.)
 template <int CTRL>
-__device__ __forceinline__ int dpp_i32(int v) { return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, false); }
+__device__ __forceinline__ int dpp_i32(int v) { return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true); }
 template <int CTRL>
 __device__ __forceinline__ float dpp_f32(float v) { return __builtin_bit_cast(float, dpp_i32<CTRL>(__builtin_bit_cast(int, v))); }
 template <int CTRL>
