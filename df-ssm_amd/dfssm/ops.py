@@ -12,6 +12,8 @@ from . import _C
 
 
 def _need(t: torch.Tensor, dtype, name: str):
+    if isinstance(t, torch.Tensor) and t.is_cuda and t.dtype is dtype:
+        return
     if not isinstance(t, torch.Tensor) or t.device.type != "cuda":
         raise TypeError(f"{name} must be a CUDA (HIP) tensor")
     if t.dtype != dtype:
@@ -48,8 +50,8 @@ _scaffold_ws = {}
 def scaffold_workspace(device) -> torch.Tensor:
     """The exchange workspace of dfssm_scaffold_lora_gemm for `device` (zeroed at allocation, one
     per device; calls on one device are ordered by torch's current stream)."""
-    dev = torch.device(device)
-    key = (dev.type, dev.index if dev.index is not None else torch.cuda.current_device())
+    dev = device if isinstance(device, torch.device) else torch.device(device)
+    key = dev.index if dev.index is not None else torch.cuda.current_device()
     if key not in _scaffold_ws:
         _scaffold_ws[key] = torch.zeros(SCAFFOLD_WORKSPACE_BYTES // 4, dtype=torch.int32, device=dev)
     return _scaffold_ws[key]
