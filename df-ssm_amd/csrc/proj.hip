@@ -211,6 +211,7 @@ __global__ __launch_bounds__(kPT) void prep_kernel(PrepArgs a, int M) {
 // 4096 and 2048 (63 workgroups: one round).
 // ------------------------------------------------------------------------------------------
 constexpr int kPrepRowsT = 1024;
+constexpr int kPrepFewRows = 1024;  // rows up to which prep_few_rows_kernel is launched
 typedef double prep_v4d __attribute__((ext_vector_type(4)));
 
 template <int KB>
@@ -324,6 +325,118 @@ __global__ __launch_bounds__(kPrepRowsT) void prep_rows_kernel(PrepArgs a, int M
     for (int i = 0; i < 16; ++i) h += part_h[256 * i + tid];
     const int row = m0 + ((tid & 63) >> 4) + 4 * (tid >> 6);
     if (row < M) a.h_out[(size_t)row * DFSSM_LORA_R + (tid & 15)] = r16((float)h);
+  }
+}
+
+// prep_few_rows_kernel<K / 512>: the same outputs with four rows per workgroup, for row counts whose
+// 16-row workgroups would leave most CUs idle. Four waves share a row (chunks of 512 columns dealt in
+// turn, two exchanges through LDS), and the LoRA contraction of 4 rows x 16 ranks runs on
+// v_mfma_f64_4x4x4_4b (the four blocks are four ranks each on the same rows), whose rate is the 16 x 16
+// instruction's at a quarter of the rows; q goes straight to its place, 64 contiguous bytes per step and
+// group.
+template <int KB>
+__global__ __launch_bounds__(kPrepRowsT) void prep_few_rows_kernel(PrepArgs a, int M) {
+  constexpr int K = 512 * KB, KW = (KB + 3) / 4;  // chunks per wave at most
+  constexpr int XS = 2 * K + 16;                  // LDS bytes of a row of xn (padded)
+  __shared__ __attribute__((aligned(16))) uint8_t xn[4 * XS];
+  __shared__ double red_d[16], part_h[16][64];
+  __shared__ float red_f[16];
+  __shared__ int red_i[16];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r4 = w & 3, qd = w >> 2;  // row of the workgroup; chunks qd, qd + 4, ...
+  const int m0 = (int)blockIdx.x * 4, m = m0 + r4;
+  const bool live = m < M;
+  const uint16_t* act = a.act + (size_t)(live ? m : M - 1) * a.ld_act + 8 * lane;
+  u32x4 v[KW];
+#pragma unroll
+  for (int i = 0; i < KW; ++i) v[i] = *(const u32x4*)(act + 512 * (qd + 4 * i < KB ? qd + 4 * i : KB - 1));
+  // this lane's LoRA-B vectors (rank lane % 16), under the norm and the quantizer
+  const int li = lane & 15, g = lane >> 4;
+  u32x4 bv[KB];
+#pragma unroll
+  for (int j = 0; j < KB; ++j) bv[j] = *(const u32x4*)(a.lBq + (size_t)li * K + 512 * j + 32 * w + 8 * g);
+  asm volatile("" ::: "memory");  // issued here, not sunk to their use
+  double part = 0.0;
+#pragma unroll
+  for (int i = 0; i < KW; ++i) {
+    if (qd + 4 * i >= KB) break;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const double x = (double)h2f((uint16_t)(v[i][e >> 1] >> (16 * (e & 1))));
+      part = __builtin_fma(x, x, part);  // (x x is exact)
+    }
+  }
+  part = wave_sum_dpp_f64(part);
+  if (lane == 0) red_d[w] = part;
+  lds_barrier();
+  const double ss = (red_d[r4] + red_d[r4 + 4]) + (red_d[r4 + 8] + red_d[r4 + 12]);
+  const float r = 1.0f / sqrt_rn((float)ss * (1.0f / (float)K) + 1e-5f);
+  float mx = 0.0f;
+#pragma unroll
+  for (int i = 0; i < KW; ++i) {
+    const int j = qd + 4 * i;
+    if (j >= KB) break;
+    const f32x4 w0 = *(const f32x4*)(a.norm_w + 512 * j + 8 * lane);
+    const f32x4 w1 = *(const f32x4*)(a.norm_w + 512 * j + 8 * lane + 4);
+    const float wv[8] = {w0[0], w0[1], w0[2], w0[3], w1[0], w1[1], w1[2], w1[3]};
+#pragma unroll
+    for (int e = 0; e < 8; e += 2) {
+      const uint32_t x2 = v[i][e >> 1];
+      const float x0 = r16((h2f((uint16_t)x2) * r) * wv[e]);
+      const float x1 = r16((h2f((uint16_t)(x2 >> 16)) * r) * wv[e + 1]);
+      mx = fmaxf(mx, fmaxf(fabsf(x0), fabsf(x1)));
+      v[i][e >> 1] = (uint32_t)f2h(x0) | ((uint32_t)f2h(x1) << 16);
+    }
+    *(u32x4*)&xn[r4 * XS + 1024 * j + 16 * lane] = v[i];
+  }
+  mx = wave_max_dpp_f32(mx);
+  if (lane == 0) red_f[w] = mx;
+  lds_barrier();  // also publishes xn
+  const float xs = quant_scale(fmaxf(fmaxf(red_f[r4], red_f[r4 + 4]), fmaxf(red_f[r4 + 8], red_f[r4 + 12])));
+  const float rinv = quant_rcp(xs);
+  double acc = 0.0;
+#pragma unroll
+  for (int j = 0; j < KB; ++j) {
+    const u32x4 av = *(const u32x4*)&xn[(lane & 3) * XS + 1024 * j + 2 * (32 * w + 8 * g)];
+#pragma unroll
+    for (int s = 0; s < 8; ++s)
+      acc = __builtin_amdgcn_mfma_f64_4x4x4f64((double)h2f((uint16_t)(av[s >> 1] >> (16 * (s & 1)))),
+                                               (double)h2f((uint16_t)(bv[j][s >> 1] >> (16 * (s & 1)))), acc, 0, 0, 0);
+  }
+  part_h[w][lane] = acc;  // row lane / 16, rank lane % 16
+  int qsum = 0;
+#pragma unroll
+  for (int i = 0; i < KW; ++i) {
+    const int j = qd + 4 * i;
+    if (j >= KB) break;
+    uint32_t qw[2] = {0u, 0u};
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int q = quant_i8(h2f((uint16_t)(v[i][e >> 1] >> (16 * (e & 1)))), rinv);
+      qw[e >> 2] |= (uint32_t)(q & 0xff) << (8 * (e & 3));
+    }
+    const int b = lane & 3, d = (lane >> 2) & 3;
+    int8_t* qt = a.q_out + (size_t)(m & ~15) * K;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      qsum = __builtin_amdgcn_sdot4((int)qw[h], 0x01010101, qsum, false);
+      const uint32_t t = quad_transpose_bytes(qw[h], b);
+      if (live) *(uint32_t*)(qt + ((8 * j + b + 4 * h) * 64 + 16 * g + (m & 15)) * 16 + 4 * d) = t;
+    }
+  }
+  const int S = wave_sum_dpp_i32(qsum);
+  if (lane == 0) red_i[w] = S;
+  lds_barrier();
+  if (qd == 0 && lane == 0 && live) {
+    a.xs_out[m] = xs;
+    a.s_out[m] = (red_i[r4] + red_i[r4 + 4]) + (red_i[r4 + 8] + red_i[r4 + 12]);
+  }
+  if (tid < 64) {
+    double h = 0.0;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) h += part_h[i][lane];
+    if (m0 + g < M) a.h_out[(size_t)(m0 + g) * DFSSM_LORA_R + li] = r16((float)h);
   }
 }
 
@@ -960,10 +1073,17 @@ hipError_t launch_prep(const PrepArgs& a, int M, int mode, hipStream_t s) {
     if (mode != DFSSM_MODE_IN || !a.lBq || !a.h_out || !a.q_out || !a.s_out || !a.xs_out || a.planes_out || a.xn_out ||
         a.xs16_out)
       return hipErrorInvalidValue;
-    const dim3 g((M + 15) / 16);
+    // four rows per workgroup while that is one round of the CUs: 999 rows 12.5 -> 8.1 us at K = 2048,
+    // 22.1 -> 13.2 at 4096, 26.6 -> 15.9 at 5120 (63 workgroups of 16 rows before); at 1280 rows both
+    // take 12.5 and 22 us, at 3072 16 rows take 13.3 and 23.5 against 18.0 and 31.5
+    const bool few = M <= kPrepFewRows;
+    const dim3 g(few ? (M + 3) / 4 : (M + 15) / 16);
     switch (a.K / 512) {
-#define DFSSM_PREP_KB(kb) \
-  case kb: hipLaunchKernelGGL((prep_rows_kernel<kb>), g, dim3(kPrepRowsT), 0, s, a, M); break;
+#define DFSSM_PREP_KB(kb)                                                                     \
+  case kb:                                                                                    \
+    if (few) hipLaunchKernelGGL((prep_few_rows_kernel<kb>), g, dim3(kPrepRowsT), 0, s, a, M); \
+    else hipLaunchKernelGGL((prep_rows_kernel<kb>), g, dim3(kPrepRowsT), 0, s, a, M);         \
+    break;
       DFSSM_PREP_KB(1) DFSSM_PREP_KB(2) DFSSM_PREP_KB(3) DFSSM_PREP_KB(4) DFSSM_PREP_KB(5)
       DFSSM_PREP_KB(6) DFSSM_PREP_KB(7) DFSSM_PREP_KB(8) DFSSM_PREP_KB(9) DFSSM_PREP_KB(10)
 #undef DFSSM_PREP_KB
