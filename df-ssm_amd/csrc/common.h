@@ -73,6 +73,32 @@ __device__ __forceinline__ float dev_expf(float x) {
   return p * sc;
 }
 
+// The sigmoid 1 / (1 + dev_expf(-x)) of x for the SiLU and the gate, in 23 instructions instead of 40.
+// -x is clamped to [-86, 87]: below, the sum is 1 as it is at -86; above, the result is 0 here where the
+// formula gives at most 2^-125, which x times it, or its own rounding to fp16, takes to zero all the
+// same. So the exponential needs no range checks, and 1 / s for 1 <= s < 2^126 is the hardware
+// reciprocal after one fma step (correctly rounded: compared with the division on every s). Compared
+// on the GPU on all 2^32 x: fp16(x sigmoid(x)) and fp16(sigmoid(x)) have the formula's bits (a NaN stays
+// a NaN).
+__device__ __forceinline__ float dev_sigmoid(float x) {
+  const float v = __builtin_amdgcn_fmed3f(-x, -86.0f, 87.0f);
+  const float n = __builtin_rintf(v * 1.44269502f);
+  float r = __builtin_fmaf(n, -0.693145751953125f, v);
+  r = __builtin_fmaf(n, -1.42860677e-6f, r);
+  float p = 1.98412698e-4f;
+  p = __builtin_fmaf(p, r, 1.38888889e-3f);
+  p = __builtin_fmaf(p, r, 8.33333333e-3f);
+  p = __builtin_fmaf(p, r, 4.16666667e-2f);
+  p = __builtin_fmaf(p, r, 1.66666667e-1f);
+  p = __builtin_fmaf(p, r, 0.5f);
+  p = __builtin_fmaf(p, r, 1.0f);
+  p = __builtin_fmaf(p, r, 1.0f);
+  const float s = 1.0f + p * __builtin_bit_cast(float, (uint32_t)((int)n + 127) << 23);
+  const float y = __builtin_amdgcn_rcpf(s);
+  const float q = __builtin_fmaf(__builtin_fmaf(-s, y, 1.0f), y, y);
+  return -x > 87.0f ? 0.0f : q;
+}
+
 __device__ __forceinline__ float dev_log_pos(float u) {  // finite u >= 1
   const uint32_t b = __builtin_bit_cast(uint32_t, u);
   int e = (int)(b >> 23) - 127;

@@ -526,7 +526,7 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& a, const GemmPro& p) {
             o = o + h2f(s2) * h2f((uint16_t)c23);
             o = o + xv * h2f((uint16_t)(c23 >> 16));
             o = o + h2f(cb ^ (uint16_t)zero);
-            const float sig = 1.0f / (1.0f + dev_expf(-o));
+            const float sig = dev_sigmoid(o);
             out = o * sig;
           }
           *op = f2h(out);

@@ -30,9 +30,11 @@ typedef u32x4 u32x4_a2 __attribute__((aligned(2)));
 // three raw inputs before its first token re-read from the rows (or the conv state). The tokens
 // of a sequence are independent once the raw rows are kept, so they spread over the grid: a thread
 // that walked the whole sequence with the outputs in place took 208 us for 999 tokens of one
-// sequence at the 1.3B shape (17 workgroups on the chip), this one 18 us. The first token range also writes the new
+// sequence at the 1.3B shape (17 workgroups on the chip), this one 13 us. The first token range also writes the new
 // conv state, the last three raw inputs. The last block of the x grid computes the decay factors of
-// its tokens, one (token, head) per thread.
+// its tokens, one (token, head) per thread. VALU issue and the rows' traffic take about the same time (36
+// instructions per value, 20 of them the exponential and the reciprocal; 133 us for 16 384 rows of the 2.7B
+// shape, 71 us at the rate of a copy).
 // ------------------------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void conv_tokens_kernel(ConvTokArgs a) {
   const int tid = threadIdx.x, b = blockIdx.z;
@@ -92,27 +94,39 @@ __global__ __launch_bounds__(256) void conv_tokens_kernel(ConvTokArgs a) {
   const bool is_x = ch < a.DI;  // (DI is a multiple of 8)
   uint16_t* out = is_x ? a.x_out + row0 * a.DI + ch : a.bc_out + row0 * (a.C - a.DI) + (ch - a.DI);
   const int ld_out = is_x ? a.DI : a.C - a.DI;
-  u32x4 nx = *(const u32x4*)(raw + (size_t)t0 * a.ld);
-  for (int t = t0; t < t1; ++t) {
-    const u32x4 v = nx;
-    nx = *(const u32x4*)(raw + (size_t)(t + 1 < t1 ? t + 1 : t) * a.ld);
-    u32x4 o = {0u, 0u, 0u, 0u};
+  // four tokens at a time, the next four on their way (tc is a multiple of four; clamped past the end)
+  constexpr int U = 4;
+  u32x4 cur[U], nx[U];
+  auto load = [&](u32x4 (&v)[U], int t) {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const uint16_t xo = (uint16_t)(v[e >> 1] >> (16 * (e & 1)));
-      const uint32_t w01 = wr[e >> 1][2 * (e & 1)], w23 = wr[e >> 1][2 * (e & 1) + 1];
-      float f = h2f(s[0][e]) * h2f((uint16_t)w01);
-      f = f + h2f(s[1][e]) * h2f((uint16_t)(w01 >> 16));
-      f = f + h2f(s[2][e]) * h2f((uint16_t)w23);
-      f = f + h2f(xo) * h2f((uint16_t)(w23 >> 16));
-      f = f + h2f((uint16_t)(br[e >> 1] >> (16 * (e & 1))));
-      const float sig = 1.0f / (1.0f + dev_expf(-f));
-      o[e >> 1] |= (uint32_t)f2h(f * sig) << (16 * (e & 1));
-      s[0][e] = s[1][e];
-      s[1][e] = s[2][e];
-      s[2][e] = xo;
+    for (int u = 0; u < U; ++u) v[u] = *(const u32x4*)(raw + (size_t)(t + u < t1 ? t + u : t1 - 1) * a.ld);
+  };
+  load(nx, t0);
+  for (int t = t0; t < t1; t += U) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) cur[u] = nx[u];
+    load(nx, t + U);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const u32x4 v = cur[u];
+      u32x4 o = {0u, 0u, 0u, 0u};
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const uint16_t xo = (uint16_t)(v[e >> 1] >> (16 * (e & 1)));
+        const uint32_t w01 = wr[e >> 1][2 * (e & 1)], w23 = wr[e >> 1][2 * (e & 1) + 1];
+        float f = h2f(s[0][e]) * h2f((uint16_t)w01);
+        f = f + h2f(s[1][e]) * h2f((uint16_t)(w01 >> 16));
+        f = f + h2f(s[2][e]) * h2f((uint16_t)w23);
+        f = f + h2f(xo) * h2f((uint16_t)(w23 >> 16));
+        f = f + h2f((uint16_t)(br[e >> 1] >> (16 * (e & 1))));
+        const float sig = dev_sigmoid(f);
+        o[e >> 1] |= (uint32_t)f2h(f * sig) << (16 * (e & 1));
+        s[0][e] = s[1][e];
+        s[1][e] = s[2][e];
+        s[2][e] = xo;
+      }
+      if (t + u < t1) *(u32x4*)(out + (size_t)(t + u) * ld_out) = o;
     }
-    *(u32x4*)(out + (size_t)t * ld_out) = o;
   }
 }
 
@@ -132,9 +146,9 @@ __global__ __launch_bounds__(256) void conv_tokens_kernel(ConvTokArgs a) {
 //   tokens on full waves.
 // Measured per layer, against the map this replaces (ssm_kernel's own, two rows and four columns per
 // lane, whose reductions took two thirds of the instructions and which kept a head on one CU):
-// 4796 -> 1483 us at the 2.7B shape and 64 x 256 tokens (1.07 ms if the four instructions per
+// 4796 -> 1449 us at the 2.7B shape and 64 x 256 tokens (1.07 ms if the four instructions per
 // element issued back to back; a wave-token takes 680 clocks of its SIMD for about 165 instructions),
-// 916 -> 150 us at the 1.3B shape and 1 x 999 tokens, 32.6 -> 8.4 us at 1 x 32 (W = 8).
+// 916 -> 147 us at the 1.3B shape and 1 x 999 tokens, 32.6 -> 8.4 us at 1 x 32 (W = 8).
 //
 // The readout's sum is ssm_kernel's tree: quads A_j of four columns summed in order from zero (the
 // product C h is exact in fp64, so an fma rounds as its multiply-then-add), Q_i = (A_4i + A_4i+1) +
@@ -398,7 +412,7 @@ __global__ __launch_bounds__(64 * W * RB, 4) void ssm_scan_kernel(ScanArgs a) {
     auto finish = [&](double s, int k) {  // item k of this thread from its row's readout
       const int t = scan_item_token<W, RB>(k);
       const float z = h2f(cur.z[k]);
-      const float sz = r16(z * r16(1.0f / (1.0f + dev_expf(-z))));
+      const float sz = r16(z * r16(dev_sigmoid(z)));
       const float y = r16((float)s + h2f(cur.x[k]) * Dh);
       if (t < nt) a.xg[((size_t)b * a.T + t0 + t) * (a.H * a.P) + col0 + scan_item_row<W, RB>()] = f2h(y * sz);
     };

@@ -579,7 +579,7 @@ __global__ __launch_bounds__(kNT) void proj_kernel(ProjArgs a) {
         o = o + h2f(cs2) * h2f((uint16_t)cw23);
         o = o + xv * h2f((uint16_t)(cw23 >> 16));
         o = o + h2f(cb);
-        const float sig = 1.0f / (1.0f + dev_expf(-o));
+        const float sig = dev_sigmoid(o);
         out = o * sig;
       }
       a.out[(size_t)m * a.ld_out + n] = f2h(out);

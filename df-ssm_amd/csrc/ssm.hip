@@ -57,8 +57,8 @@ __device__ __forceinline__ void ssm_rows(const SsmArgs& a, int bx, int m, uint32
   float sz0 = 0.0f, sz1 = 0.0f;
   if (GATE) {
     const float z0 = h2f(zr0), z1 = h2f(zr1);
-    sz0 = r16(z0 * r16(1.0f / (1.0f + dev_expf(-z0))));
-    sz1 = r16(z1 * r16(1.0f / (1.0f + dev_expf(-z1))));
+    sz0 = r16(z0 * r16(dev_sigmoid(z0)));
+    sz1 = r16(z1 * r16(dev_sigmoid(z1)));
   }
   const uint32_t bw[2] = {b4.x, b4.y}, cw[2] = {c4.x, c4.y};
   float h0[4] = {s0.x, s0.y, s0.z, s0.w}, h1[4] = {s1.x, s1.y, s1.z, s1.w};
@@ -289,7 +289,7 @@ __global__ __launch_bounds__(256) void conv_kernel(ConvArgs a) {
   o = o + s2 * h2f(wc[2]);
   o = o + xv * h2f(wc[3]);
   o = o + h2f(a.b[ch]);
-  const float sig = 1.0f / (1.0f + dev_expf(-o));
+  const float sig = dev_sigmoid(o);
   *xp = f2h(o * sig);
 }
 
