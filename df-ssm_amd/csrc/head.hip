@@ -71,17 +71,17 @@ __device__ __forceinline__ void wave_argmax_dpp(float& b, int& bi) {
 }
 
 // The last workgroup's argmax over the NG per-workgroup (max, first index) pairs of every row
-// (part_val/part_idx, row-major by row): wave w takes rows w + NWV (r0 + r), r < RW, and every
+// (part_val/part_idx, row-major by row): wave w takes rows w + NWV r, r < RW, and every
 // lane loads all its pairs of all those rows (at most K each, clamped in-bounds addresses) before
-// comparing any, so the reduction costs one memory round trip. Writes a.next and toks.
+// comparing any, so the reduction costs one memory round trip. Writes a.next and, if given, toks.
 template <int NWV, int RW, int K>
-__device__ __forceinline__ void argmax_pairs(const HeadArgs& a, int M, int NG, int* toks, int r0 = 0) {
+__device__ __forceinline__ void argmax_pairs(const HeadArgs& a, int M, int NG, int* toks = nullptr) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   float pv[RW][K];
   int pi[RW][K];
 #pragma unroll
   for (int r = 0; r < RW; ++r) {
-    const int m = wave + NWV * (r0 + r) < M ? wave + NWV * (r0 + r) : M - 1;
+    const int m = wave + NWV * r < M ? wave + NWV * r : M - 1;
 #pragma unroll
     for (int q = 0; q < K; ++q) {
       const int j = lane + 64 * q < NG ? lane + 64 * q : NG - 1;
@@ -91,7 +91,7 @@ __device__ __forceinline__ void argmax_pairs(const HeadArgs& a, int M, int NG, i
   }
 #pragma unroll
   for (int r = 0; r < RW; ++r) {
-    const int m = wave + NWV * (r0 + r);
+    const int m = wave + NWV * r;
     float b = -INFINITY;
     int bi = 0x7fffffff;
 #pragma unroll
@@ -105,7 +105,7 @@ __device__ __forceinline__ void argmax_pairs(const HeadArgs& a, int M, int NG, i
       // no comparable logit (all NaN): report token 0 rather than an index outside the table
       if (bi < 0 || bi >= a.V) bi = 0;
       a.next[m] = (int64_t)bi;
-      toks[m] = bi;
+      if (toks) toks[m] = bi;
     }
   }
 }
@@ -240,16 +240,37 @@ __global__ __launch_bounds__(256) void head_kernel(HeadArgs a) {
   if (a.x_next) embed_next<F16, 256>(a, next_tok, M, D);
 }
 
-__global__ __launch_bounds__(256) void embed_kernel(EmbedArgs a) {
-  const int m = blockIdx.x;
+// x[m] = the embedding of token m: one 16-byte table chunk (16 int8 or 8 fp16 values) per thread. (A
+// value per load and store, one workgroup per row, took 78 us for 16 384 rows of the 2.7B shape; this
+// 66: the chunks of a row are 1 KiB apart in the table, so every one is a line of its own.) x needs no
+// more alignment than its elements.
+typedef u32x4 emb_u32x4_a2 __attribute__((aligned(2)));
+__global__ __launch_bounds__(256) void embed_kernel(EmbedArgs a, int M) {
+  const int CH = a.f16 ? a.D / 8 : a.D / 16;
+  const int i = (int)blockIdx.x * 256 + (int)threadIdx.x;
+  if (i >= M * CH) return;
+  const int m = i / CH, c = i - m * CH;
   const int64_t t64 = a.tok_tc > 0 ? a.tokens[(size_t)(m / a.tok_tc) * a.tok_ld + a.tok_t0 + m % a.tok_tc] : a.tokens[m];
-  const int t = (t64 < 0 || t64 >= a.V) ? 0 : (int)t64;
-  if (t64 < 0 || t64 >= a.V) {
-    if (threadIdx.x == 0) atomicOr(a.err_flag, DFSSM_ERR_TOKEN_RANGE);
+  const bool bad = t64 < 0 || t64 >= a.V;
+  const int t = bad ? 0 : (int)t64;
+  if (bad && c == 0) atomicOr(a.err_flag, DFSSM_ERR_TOKEN_RANGE);
+  const u32x4 ch = *(const u32x4*)(a.emb + (((size_t)(t >> 6) * CH + c) * 64 + (t & 63)) * 16);
+  if (a.f16) {
+    *(emb_u32x4_a2*)(a.x + (size_t)m * a.D + 8 * c) = ch;
+    return;
   }
-  for (int k = threadIdx.x; k < a.D; k += 256)
-    a.x[(size_t)m * a.D + k] = a.f16 ? emb_value<true>(a.emb, a.emb_scale, a.D / 8, t >> 6, t & 63, k)
-                                     : emb_value<false>(a.emb, a.emb_scale, a.D / 16, t >> 6, t & 63, k);
+  const float sv = h2f(a.emb_scale[t]);
+  u32x4 o[2];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const uint32_t w = ch[e >> 1];
+    const int sh = 16 * (e & 1);
+    const float v0 = (float)(int8_t)(w >> sh) * sv, v1 = (float)(int8_t)(w >> (sh + 8)) * sv;
+    o[e >> 2][e & 3] = (uint32_t)f2h(v0) | ((uint32_t)f2h(v1) << 16);
+  }
+  emb_u32x4_a2* dst = (emb_u32x4_a2*)(a.x + (size_t)m * a.D + 16 * c);
+  dst[0] = o[0];
+  dst[1] = o[1];
 }
 
 // Re-tile a row-major (V, D) table of D bytes per row into [V_pad/64][D/16][64][16].
@@ -548,7 +569,8 @@ hipError_t launch_head(const HeadArgs& a, int M, hipStream_t s) {
 }
 
 hipError_t launch_embed(const EmbedArgs& a, int M, hipStream_t s) {
-  hipLaunchKernelGGL(embed_kernel, dim3(M), dim3(256), 0, s, a);
+  const long long n = (long long)M * (a.f16 ? a.D / 8 : a.D / 16);
+  hipLaunchKernelGGL(embed_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a, M);
   return hipGetLastError();
 }
 
@@ -679,7 +701,6 @@ __global__ __launch_bounds__(kHsThreads) __attribute__((amdgpu_waves_per_eu(2)))
   __shared__ float wbest[kHsWaves][16 * NHW];
   __shared__ int widx[kHsWaves][16 * NHW];
   __shared__ bool is_last;
-  __shared__ int next_tok[MP];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int rg = wave / WPG, wf = wave % WPG;     // row group, fragment slot
@@ -847,12 +868,8 @@ __global__ __launch_bounds__(kHsThreads) __attribute__((amdgpu_waves_per_eu(2)))
   if (tid == 0) is_last = atomicAdd(a.ticket, 1u) == (unsigned)(NGW - 1);
   __syncthreads();
   if (!is_last) return;
-  argmax_pairs<kHsWaves, (MP + kHsWaves - 1) / kHsWaves, kHeadMaxGroups / 128>(a, M, NGW, next_tok);
+  argmax_pairs<kHsWaves, (MP + kHsWaves - 1) / kHsWaves, kHeadMaxGroups / 128>(a, M, NGW);
   if (tid == 0) *a.ticket = 0u;
-  __syncthreads();
-  // the embedding in one round of loads up to 20 chunks per thread (64 rows of 2560 bytes)
-  constexpr int KBE = (MP * 320 + kHsThreads - 1) / kHsThreads < 20 ? (MP * 320 + kHsThreads - 1) / kHsThreads : 20;
-  if (a.x_next) embed_next<false, kHsThreads, KBE>(a, next_tok, M, D);
 }
 
 template <int NH>
@@ -877,9 +894,9 @@ static hipError_t launch_head_i8s(const HeadArgs& a, int M, hipStream_t s) {
 // loop waits for more than the oldest step. xf goes through LDS 512 columns at a time, double-buffered,
 // the next chunk loaded under the current one. Measured at the 2.7B shape and 64 rows against 4 waves
 // of 64 vocabulary rows with two steps in flight and xf staged behind two full barriers per chunk:
-// 233 -> 111 us in the decode step (where the state stream's dirty lines leave the last-level cache
-// under it), 85 us back to back (3.1 TB/s; 58 us at 5 rows, 4.4 TB/s). 4 or 16 steps in flight measure
-// the same, temporal loads 92 us.
+// 233 -> 67 us in the decode step, 3.8 TB/s (111 us with the next tokens' embeddings gathered by the last
+// workgroup, as in the 233). Back to back 4 or 16 steps in flight, or two or four table tiles per wave
+// (fewer LDS reads), measure the same; temporal loads are 9% slower.
 // Argmax as above: per-workgroup pairs, then the last workgroup to finish reduces them.
 // ---------------------------------------------------------------------------------------------
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
@@ -912,7 +929,6 @@ __global__ __launch_bounds__(kHT) void head_mfma_kernel(HeadArgs a, int M) {
   __shared__ float wbest[16][MP];
   __shared__ int widx[16][MP];
   __shared__ bool is_last;
-  __shared__ int next_tok[MP];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int lr = lane & 15, g = lane >> 4;
   const int D = a.D, CH = D / 8, NC = D / kHK;
@@ -999,27 +1015,26 @@ __global__ __launch_bounds__(kHT) void head_mfma_kernel(HeadArgs a, int M) {
   __syncthreads();
   if (!is_last) return;
   __threadfence();
-  argmax_pairs<16, MI, kHeadMaxGroups / 256>(a, M, (int)gridDim.x, next_tok);
+  argmax_pairs<16, MI, kHeadMaxGroups / 256>(a, M, (int)gridDim.x);
   if (tid == 0) *a.ticket = 0u;
-  __syncthreads();
-  if (a.x_next) embed_next<true, kHT>(a, next_tok, M, D);
 }
 
-hipError_t launch_head_batched(const HeadArgs& a, int M, hipStream_t s) {
-  if (M < 1 || M > 64 || a.D % kHK || (a.V + 63) / 64 > kHeadMaxGroups) return hipErrorInvalidValue;
-  if (!a.f16) {  // int8 table: exact digit-plane GEMM
-    if (!a.hdig) return hipErrorInvalidValue;
-    const int nh = (M + 15) / 16;
-    hipLaunchKernelGGL(head_digits_kernel, dim3(16 * nh), dim3(256), 0, s, a.x, a.norm_f, (int8_t*)a.hdig, M, nh, a.D);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    switch (nh) {
-      case 1: return launch_head_i8s<1>(a, M, s);
-      case 2: return launch_head_i8s<2>(a, M, s);
-      case 3: return launch_head_i8s<3>(a, M, s);
-      default: return launch_head_i8s<4>(a, M, s);
-    }
+// int8 table: exact digit-plane GEMM
+static hipError_t launch_head_i8(const HeadArgs& a, int M, hipStream_t s) {
+  if (!a.hdig) return hipErrorInvalidValue;
+  const int nh = (M + 15) / 16;
+  hipLaunchKernelGGL(head_digits_kernel, dim3(16 * nh), dim3(256), 0, s, a.x, a.norm_f, (int8_t*)a.hdig, M, nh, a.D);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  switch (nh) {
+    case 1: return launch_head_i8s<1>(a, M, s);
+    case 2: return launch_head_i8s<2>(a, M, s);
+    case 3: return launch_head_i8s<3>(a, M, s);
+    default: return launch_head_i8s<4>(a, M, s);
   }
+}
+
+static hipError_t launch_head_f16(const HeadArgs& a, int M, hipStream_t s) {
   if (!a.xf) return hipErrorInvalidValue;
   hipLaunchKernelGGL(final_norm_kernel, dim3(M), dim3(256), 0, s, a.x, a.norm_f, (uint16_t*)a.xf, a.D);
   hipError_t e = hipGetLastError();
@@ -1034,6 +1049,21 @@ hipError_t launch_head_batched(const HeadArgs& a, int M, hipStream_t s) {
   DFSSM_HEAD_MFMA(4)
 #undef DFSSM_HEAD_MFMA
   return hipGetLastError();
+}
+
+hipError_t launch_head_batched(const HeadArgs& a, int M, hipStream_t s) {
+  if (M < 1 || M > 64 || a.D % kHK || (a.V + 63) / 64 > kHeadMaxGroups) return hipErrorInvalidValue;
+  const hipError_t e = a.f16 ? launch_head_f16(a, M, s) : launch_head_i8(a, M, s);
+  if (e != hipSuccess || !a.x_next) return e;
+  // The next tokens' rows, in a launch of their own: a row's 16-byte chunks are 1 KiB apart in the table,
+  // and one CU (the head's last workgroup, as for up to four rows) gathers 64 rows of a 2560-column fp16
+  // table in 13 us, three times that when the state stream has evicted the table. Decode step of two
+  // such layers at 64 rows 333 -> 281 us; 48 layers at 32 rows (int8) 2206 -> 2189; 16 layers at 5, 8 and 16
+  // rows 450, 484 and 584 us both ways (int8), 459, 507 and 607 -> 457, 504 and 598 (fp16).
+  EmbedArgs em{};  // (every next token is in range: no error flag)
+  em.tokens = a.next; em.emb = a.emb; em.emb_scale = a.emb_scale; em.f16 = a.f16; em.x = a.x_next;
+  em.V = a.V; em.D = a.D;
+  return launch_embed(em, M, s);
 }
 
 }  // namespace dfssm
