@@ -123,3 +123,24 @@ def test_conv_ssm_128_steps(B):
     np.testing.assert_array_equal(_np16(g_conv).view(np.uint16), r_conv.view(np.uint16))
     for gy, ry in ys:
         assert np.abs(gy - ry).max() <= 1e-3 * np.abs(ry).max() + 1e-3
+
+
+@pytest.mark.parametrize("w3", [1.0, 37.0, 65504.0])
+def test_silu_all_halves(w3):
+    """SiLU of every fp16 value (times a conv weight: sums up to 4.3e9, infinities and NaN) against the
+    oracle's formula, bit for bit: the clamped exponential and the reciprocal of the kernels."""
+    x = np.arange(65536, dtype=np.uint16).view(np.float16).reshape(1, -1)
+    C = x.shape[1]
+    w = np.zeros((C, 4), np.float16)
+    w[:, 3] = w3
+    b = np.zeros(C, np.float16)
+    st = np.zeros((1, C, 3), np.float16)
+    print(f"silu of all halves times {w3}", flush=True)
+    gx = _h(x)
+    ops.conv_step(_h(st), gx, _h(w), _h(b))
+    rx = x.copy()
+    O.conv_step(st.copy(), rx, w, b)
+    got = _np16(gx)
+    nan = np.isnan(rx)
+    np.testing.assert_array_equal(np.isnan(got), nan)
+    np.testing.assert_array_equal(got.view(np.uint16)[~nan], rx.view(np.uint16)[~nan])
