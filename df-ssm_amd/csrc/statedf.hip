@@ -80,14 +80,21 @@ __global__ __launch_bounds__(32 * kDfRows) void state_df_kernel(StateDfArgs a, i
     const float range = t6 > 1e-8f ? t6 : 1e-8f;
     // num / range for all values of the row as one product each: in fp64 num * RN(1 / range) is within
     // 2^-52 of the quotient, and a quotient of two fp32 values is at least 2^-49 (relative) away from
-    // any midpoint of neighbouring fp32 values, so both round to the same fp32 value
+    // any midpoint of neighbouring normal fp32 values, so both round to the same fp32 value. A subnormal
+    // quotient can be a tie; it needs lo = 0 (else num is 0 or at least 2^-50 range): that row divides
     const double rinv = 1.0 / (double)range;
-    float hc[4], out[4], err[4];
+    const bool any0 = __builtin_expect(__builtin_amdgcn_ballot_w64(lo == 0.0f) != 0, 0);  // uniform
+    float quo[4], hc[4], out[4], err[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) quo[k] = (float)((double)(hv[k] - lo) * rinv);
+    if (any0) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) quo[k] = lo == 0.0f ? (hv[k] - lo) / range : quo[k];
+    }
     uint32_t first[4];  // number of thresholds below hc, times 4
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      const float num = hv[k] - lo;
-      float hs = (float)((double)num * rinv);
+      float hs = quo[k];
       hs = hs < 0.0f ? 0.0f : (hs > 1.0f ? 1.0f : hs);
       hc[k] = hs;
       if (ERR) {

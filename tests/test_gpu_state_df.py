@@ -59,6 +59,28 @@ def test_kernel_vs_oracle(kk, sd, bits):
         h, e = ho, eo
 
 
+@pytest.mark.parametrize("bits", [8, 32])
+def test_subnormal_quotients(bits):
+    """A row whose mean is three times its deviation (lo = 0, range 98) with subnormal values: quotients
+    that are ties of subnormals, where a product with the rounded reciprocal rounds the other way."""
+    h = np.zeros((16, 128), np.float32)
+    h[:, :115] = np.float32(54.464615)
+    h[:, 115] = np.float32(8.569192886352539)
+    h[:, 116:] = (np.uint32(49) * np.arange(1, 193, dtype=np.uint32)).reshape(16, 12).view(np.float32)
+    num = h[:, 116:]
+    assert (num / np.float32(98) != (num.astype(np.float64) * (1.0 / 98.0)).astype(np.float32)).any()
+    e = np.zeros_like(h)
+    R = np.linspace(0.01, 1, 64, dtype=np.float32)
+    ho, eo = O.state_density_field(h, R, e, bits)
+    assert (ho[:, 116:] == 0).all()  # lo
+    if bits == 32:
+        np.testing.assert_array_equal(eo[:, 116:], num / np.float32(98))  # range
+    print(f"state df subnormal quotients bits={bits}", flush=True)
+    hg, eg = _gpu_df(h, R, e, bits)
+    np.testing.assert_array_equal(hg.view(np.uint32), ho.view(np.uint32))
+    np.testing.assert_array_equal(eg.view(np.uint32), eo.view(np.uint32))
+
+
 def test_full_size_state():
     """The 1.3B state at batch 1 (48 x 64 x 64 rows) in one call."""
     rng = np.random.default_rng(1)
