@@ -1,8 +1,8 @@
 """ctypes binding of libdfssm_hip.so (declarations: include/dfssm.h).
 
 Only plain pointers, sizes and the stream cross the boundary; torch tensors are unpacked here
-with data_ptr() and torch.cuda.current_stream().cuda_stream, so every launch lands on the
-caller's current stream and can be captured into a HIP graph. There is no fallback: if the
+with data_ptr() and stream() passes torch's current stream, so every launch lands on the caller's
+current stream and can be captured into a HIP graph. There is no fallback: if the
 library is missing or a call fails, an exception is raised.
 """
 from __future__ import annotations
@@ -124,11 +124,20 @@ def ptr(t) -> int:
 _get_raw_stream = None
 
 
+def _forget_stream_getter() -> None:
+    global _get_raw_stream
+    _get_raw_stream = None
+
+
+os.register_at_fork(after_in_child=_forget_stream_getter)
+
+
 def stream() -> int:
     """torch's current stream of the current device, as a hipStream_t. The first call goes through
     torch.cuda.current_stream() (which initialises the device); that builds a Stream object behind
     a dozen Python calls each time, 6 of the 14.6 us of a single-operator call, so later calls ask
-    torch's C layer for the same handle."""
+    torch's C layer for the same handle. A forked child asks torch again, which refuses to use the
+    parent's GPU context there."""
     global _get_raw_stream
     import torch
     if _get_raw_stream is None:

@@ -1,6 +1,8 @@
 """Host-side logic of the drop-in API, checked without a GPU: the one-launch layer's residency
 rule (dfssm_one_launch_plan), the decoding of the workspace error flag, and token range checks that
 must fire before any kernel reads the ids."""
+import os
+
 import numpy as np
 import pytest
 import torch
@@ -92,3 +94,30 @@ def test_generate_checks_prompt_shape():
     m = _hostless_model(B=2)
     with pytest.raises(ValueError):
         m.generate(n_tokens=4, prompt=torch.zeros(3, 2, dtype=torch.int64), verbose=False)
+
+
+def test_stream_in_forked_child_asks_torch_again(monkeypatch):
+    """A process that has launched work asks torch's C layer for the stream directly; a child forked from it
+    goes through torch.cuda again, whose error for a forked GPU context must reach the caller."""
+    class Stream:
+        cuda_stream = 7
+
+    monkeypatch.setattr(_C, "_get_raw_stream", None)
+    monkeypatch.setattr(torch.cuda, "current_stream", Stream)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda device: 9, raising=False)
+    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: 0, raising=False)
+    assert (_C.stream(), _C.stream()) == (7, 9)
+
+    def refuse():
+        raise RuntimeError("Cannot re-initialize CUDA in forked subprocess")
+
+    monkeypatch.setattr(torch.cuda, "current_stream", refuse)
+    assert _C.stream() == 9
+    pid = os.fork()
+    if pid == 0:
+        try:
+            _C.stream()
+            os._exit(1)
+        except RuntimeError:
+            os._exit(0)
+    assert os.waitstatus_to_exitcode(os.waitpid(pid, 0)[1]) == 0
