@@ -51,7 +51,7 @@ def scaffold_workspace(device) -> torch.Tensor:
     """The exchange workspace of dfssm_scaffold_lora_gemm for `device` (zeroed at allocation, one
     per device; calls on one device are ordered by torch's current stream)."""
     dev = device if isinstance(device, torch.device) else torch.device(device)
-    key = dev.index if dev.index is not None else torch.cuda.current_device()
+    key = (dev.type, dev.index if dev.index is not None else torch.cuda.current_device())
     if key not in _scaffold_ws:
         _scaffold_ws[key] = torch.zeros(SCAFFOLD_WORKSPACE_BYTES // 4, dtype=torch.int32, device=dev)
     return _scaffold_ws[key]

@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 import torch
 
-from dfssm import _C
+from dfssm import _C, ops
 from dfssm.synth import config_tiny
 import df_ssm_inference as dfi
 
@@ -121,3 +121,12 @@ def test_stream_in_forked_child_asks_torch_again(monkeypatch):
         except RuntimeError:
             os._exit(0)
     assert os.waitstatus_to_exitcode(os.waitpid(pid, 0)[1]) == 0
+
+
+def test_scaffold_workspace_of_another_device_type(monkeypatch):
+    """A workspace asked for on another device type is not handed to the GPU's calls, nor the other way round."""
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(ops, "_scaffold_ws", type(ops._scaffold_ws)())
+    host = ops.scaffold_workspace("cpu")
+    assert host.device.type == "cpu" and ops.scaffold_workspace("cpu") is host
+    assert ops.scaffold_workspace(torch.device("meta")).device.type == "meta"
