@@ -6,6 +6,8 @@ there is no CPU fallback.
 """
 from __future__ import annotations
 
+import threading
+
 import torch
 
 from . import _C
@@ -44,17 +46,38 @@ def scaffold_gemm(tiled_bits: torch.Tensor, q: torch.Tensor, N: int, xscale=None
 
 SCAFFOLD_WORKSPACE_BYTES = 64 << 10   # DFSSM_SCAFFOLD_WORKSPACE_BYTES
 SCAFFOLD_ERROR_OFFSET = 1024          # DFSSM_SCAFFOLD_ERROR_OFFSET
+SCAFFOLD_WORKSPACE_STREAMS = 64       # streams whose workspaces are kept
 _scaffold_ws = {}
+_scaffold_ws_lock = threading.Lock()
+
+
+def _new_scaffold_workspace(device) -> torch.Tensor:
+    return torch.zeros(SCAFFOLD_WORKSPACE_BYTES // 4, dtype=torch.int32, device=device)
 
 
 def scaffold_workspace(device) -> torch.Tensor:
-    """The exchange workspace of dfssm_scaffold_lora_gemm for `device` (zeroed at allocation, one
-    per device; calls on one device are ordered by torch's current stream)."""
+    """The exchange workspace of dfssm_scaffold_lora_gemm for calls on torch's current stream of `device`,
+    zeroed on that stream at allocation. Calls that share one must not overlap, so every stream has its
+    own; those of the last SCAFFOLD_WORKSPACE_STREAMS streams are kept. A stream that is being captured
+    gets a new one at each call, owned by its graph and zeroed at every replay: a kept one would tie
+    the graph's replays to whatever runs on the capture's stream then."""
+    return _stream_workspace(device, _C.stream())
+
+
+def _stream_workspace(device, stream: int) -> torch.Tensor:
     dev = device if isinstance(device, torch.device) else torch.device(device)
-    key = (dev.type, dev.index if dev.index is not None else torch.cuda.current_device())
-    if key not in _scaffold_ws:
-        _scaffold_ws[key] = torch.zeros(SCAFFOLD_WORKSPACE_BYTES // 4, dtype=torch.int32, device=dev)
-    return _scaffold_ws[key]
+    if torch.cuda.is_current_stream_capturing():
+        return _new_scaffold_workspace(dev)
+    key = (dev.type, dev.index if dev.index is not None else torch.cuda.current_device(), stream)
+    ws = _scaffold_ws.get(key)
+    if ws is None:
+        with _scaffold_ws_lock:
+            ws = _scaffold_ws.get(key)
+            if ws is None:
+                while len(_scaffold_ws) >= SCAFFOLD_WORKSPACE_STREAMS:  # (freed in its stream's order)
+                    del _scaffold_ws[next(iter(_scaffold_ws))]
+                ws = _scaffold_ws[key] = _new_scaffold_workspace(dev)
+    return ws
 
 
 def scaffold_error(workspace: torch.Tensor) -> int:
@@ -68,8 +91,9 @@ def scaffold_lora_gemm(tiled_bits: torch.Tensor, wscale: torch.Tensor, q: torch.
     """One projection with its LoRA (dfssm_scaffold_lora_gemm): returns (acc int32 (M, N),
     y fp16 (M, N), lora_h fp16 (M, 16)). q (M, K) int8 with fp16 scales xscale (M,), xn (M, K) fp16,
     lA (N, 16) int8, lA_s (N,) fp16, lBq (16, K) fp16, wscale (N,) fp16. workspace: "auto" (the
-    device's exchange workspace: one launch at M <= 4), None (no workspace) or an int32 tensor of
-    SCAFFOLD_WORKSPACE_BYTES, zeroed before its first use."""
+    current stream's exchange workspace: one launch at M <= 4; in a capture one more, which clears it),
+    None (no workspace) or an int32 tensor of SCAFFOLD_WORKSPACE_BYTES, zeroed before its first use and
+    used by calls that do not overlap."""
     _need(q, torch.int8, "q")
     _need(xn, torch.float16, "xn")
     _need(lBq, torch.float16, "lBq")
@@ -80,10 +104,11 @@ def scaffold_lora_gemm(tiled_bits: torch.Tensor, wscale: torch.Tensor, q: torch.
     acc = torch.empty(M, N, dtype=torch.int32, device=q.device)
     y = torch.empty(M, N, dtype=torch.float16, device=q.device)
     h = torch.empty(M, 16, dtype=torch.float16, device=q.device)
+    stream = _C.stream()
     if isinstance(workspace, str):
         if workspace != "auto":
             raise ValueError('workspace must be "auto", None or a tensor')
-        workspace = scaffold_workspace(q.device)
+        workspace = _stream_workspace(q.device, stream) if M <= 4 else None  # (unused by more rows)
     elif workspace is not None:
         _need(workspace, torch.int32, "workspace")
         if workspace.numel() * 4 < SCAFFOLD_WORKSPACE_BYTES:
@@ -92,7 +117,7 @@ def scaffold_lora_gemm(tiled_bits: torch.Tensor, wscale: torch.Tensor, q: torch.
         tiled_bits.data_ptr(), wscale.contiguous().data_ptr(), q.contiguous().data_ptr(),
         xscale.contiguous().data_ptr(), xn.contiguous().data_ptr(), lA.contiguous().data_ptr(),
         lA_s.contiguous().data_ptr(), lBq.contiguous().data_ptr(), M, N, K, h.data_ptr(), acc.data_ptr(),
-        y.data_ptr(), _C.ptr(workspace), _C.stream()), "scaffold_lora_gemm")
+        y.data_ptr(), _C.ptr(workspace), stream), "scaffold_lora_gemm")
     return acc, y, h
 
 

@@ -123,10 +123,40 @@ def test_stream_in_forked_child_asks_torch_again(monkeypatch):
     assert os.waitstatus_to_exitcode(os.waitpid(pid, 0)[1]) == 0
 
 
-def test_scaffold_workspace_of_another_device_type(monkeypatch):
-    """A workspace asked for on another device type is not handed to the GPU's calls, nor the other way round."""
+@pytest.fixture
+def host_workspaces(monkeypatch):
+    """scaffold_workspace without a GPU: an empty cache, buffers on the host, a settable stream handle."""
+    real, env = torch.zeros, {"stream": 1, "capturing": False}
+    monkeypatch.setattr(torch, "zeros", lambda *a, device=None, **k: real(
+        *a, device=device if torch.device(device).type == "meta" else None, **k))
     monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: env["capturing"])
+    monkeypatch.setattr(_C, "stream", lambda: env["stream"])
     monkeypatch.setattr(ops, "_scaffold_ws", type(ops._scaffold_ws)())
+    return env
+
+
+def test_scaffold_workspace_of_another_device_type(host_workspaces):
+    """A workspace asked for on another device type is not handed to the GPU's calls, nor the other way round."""
     host = ops.scaffold_workspace("cpu")
     assert host.device.type == "cpu" and ops.scaffold_workspace("cpu") is host
     assert ops.scaffold_workspace(torch.device("meta")).device.type == "meta"
+
+
+def test_scaffold_workspace_per_stream(host_workspaces):
+    """Calls on two streams may overlap and calls that share a workspace must not: every stream has its own,
+    every call of a capture too (its graph may be replayed on any stream), and the number kept is bounded."""
+    first = ops.scaffold_workspace("cuda:0")
+    assert ops.scaffold_workspace("cuda") is first
+    host_workspaces["stream"] = 2
+    second = ops.scaffold_workspace("cuda:0")
+    assert second.data_ptr() != first.data_ptr()
+    assert ops.scaffold_workspace("cuda:1").data_ptr() != second.data_ptr()
+    host_workspaces["capturing"] = True
+    captured = [ops.scaffold_workspace("cuda:0") for _ in range(2)]
+    assert len({t.data_ptr() for t in captured + [first, second]}) == 4
+    host_workspaces["capturing"] = False
+    assert ops.scaffold_workspace("cuda:0") is second
+    for host_workspaces["stream"] in range(100, 400):
+        ops.scaffold_workspace("cuda:0")
+    assert len(ops._scaffold_ws) <= 64

@@ -106,6 +106,35 @@ def test_scaffold_lora_op_shared_workspace():
     assert (counts == one_launch).all()  # every workgroup index counted every one-launch call
 
 
+def test_scaffold_lora_op_streams_and_graphs():
+    """Calls with the automatic workspace on two streams that may overlap, and in a captured graph replayed
+    between eager calls: every result is the oracle's."""
+    cases = [_lora_op_case(8512, 2048, 1, 20), _lora_op_case(2048, 2048, 4, 21)]
+    print("scaffold+lora on two streams", flush=True)
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    outs = []
+    for _ in range(8):
+        for s, (args, _) in zip(streams, cases):
+            with torch.cuda.stream(s):
+                outs.append(ops.scaffold_lora_gemm(*args))
+    torch.cuda.synchronize()
+    for i, out in enumerate(outs):
+        _check_lora_op(out, cases[i % 2][1])
+    print("scaffold+lora in a graph", flush=True)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        captured = [ops.scaffold_lora_gemm(*args) for args, _ in cases]
+    for _ in range(4):
+        g.replay()
+        torch.cuda.synchronize()
+        for out, (_, ref) in zip(captured, cases):
+            _check_lora_op(out, ref)
+            out[1].zero_()
+        for args, ref in cases:
+            _check_lora_op(ops.scaffold_lora_gemm(*args), ref)
+
+
 # ------------------------------------------------------------------------------ config 3, B = 32
 @pytest.fixture(scope="module")
 def w13():
