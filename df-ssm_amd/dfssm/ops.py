@@ -2,7 +2,8 @@
 
 These are the operator-level entry points (scaffold GEMM, RMSNorm+quantize, conv step, SSM step,
 bit/embedding tiling). Every call launches on torch's current stream and raises on any error;
-there is no CPU fallback.
+there is no CPU fallback. Arguments that are not contiguous are copied; all copies of a call stay bound
+to names until its launch, so that the allocator cannot give one's memory to the next.
 """
 from __future__ import annotations
 
@@ -38,8 +39,9 @@ def scaffold_gemm(tiled_bits: torch.Tensor, q: torch.Tensor, N: int, xscale=None
     M, K = q.shape
     acc = torch.empty(M, N, dtype=torch.int32, device=q.device)
     y = torch.empty(M, N, dtype=torch.float16, device=q.device) if want_y else None
+    q = q.contiguous()
     _C.check(_C.lib().dfssm_scaffold_gemm(
-        tiled_bits.data_ptr(), q.contiguous().data_ptr(), _C.ptr(xscale), _C.ptr(wscale), M, N, K,
+        tiled_bits.data_ptr(), q.data_ptr(), _C.ptr(xscale), _C.ptr(wscale), M, N, K,
         acc.data_ptr(), _C.ptr(y), _C.stream()), "scaffold_gemm")
     return (acc, y) if want_y else acc
 
@@ -113,11 +115,11 @@ def scaffold_lora_gemm(tiled_bits: torch.Tensor, wscale: torch.Tensor, q: torch.
         _need(workspace, torch.int32, "workspace")
         if workspace.numel() * 4 < SCAFFOLD_WORKSPACE_BYTES:
             raise ValueError(f"workspace must hold {SCAFFOLD_WORKSPACE_BYTES} bytes")
+    wscale, q, xscale, xn = wscale.contiguous(), q.contiguous(), xscale.contiguous(), xn.contiguous()
+    lA, lA_s, lBq = lA.contiguous(), lA_s.contiguous(), lBq.contiguous()
     _C.check(_C.lib().dfssm_scaffold_lora_gemm(
-        tiled_bits.data_ptr(), wscale.contiguous().data_ptr(), q.contiguous().data_ptr(),
-        xscale.contiguous().data_ptr(), xn.contiguous().data_ptr(), lA.contiguous().data_ptr(),
-        lA_s.contiguous().data_ptr(), lBq.contiguous().data_ptr(), M, N, K, h.data_ptr(), acc.data_ptr(),
-        y.data_ptr(), _C.ptr(workspace), stream), "scaffold_lora_gemm")
+        tiled_bits.data_ptr(), wscale.data_ptr(), q.data_ptr(), xscale.data_ptr(), xn.data_ptr(), lA.data_ptr(),
+        lA_s.data_ptr(), lBq.data_ptr(), M, N, K, h.data_ptr(), acc.data_ptr(), y.data_ptr(), _C.ptr(workspace), stream), "scaffold_lora_gemm")
     return acc, y, h
 
 
@@ -129,7 +131,8 @@ def rmsnorm_quantize(x: torch.Tensor, w: torch.Tensor):
     xn = torch.empty_like(x)
     q = torch.empty(M, K, dtype=torch.int8, device=x.device)
     s = torch.empty(M, dtype=torch.float16, device=x.device)
-    _C.check(_C.lib().dfssm_rmsnorm_quantize(x.contiguous().data_ptr(), w.contiguous().data_ptr(), M, K,
+    x, w = x.contiguous(), w.contiguous()
+    _C.check(_C.lib().dfssm_rmsnorm_quantize(x.data_ptr(), w.data_ptr(), M, K,
                                              xn.data_ptr(), q.data_ptr(), s.data_ptr(), _C.stream()),
              "rmsnorm_quantize")
     return xn, q, s
@@ -144,9 +147,9 @@ def conv_step(conv_state: torch.Tensor, xbc: torch.Tensor, conv_w: torch.Tensor,
         raise ValueError(f"conv_state must be contiguous ({B}, {C}, 3)")
     if xbc.stride(1) != 1:
         raise ValueError("xBC rows must be contiguous")
-    _C.check(_C.lib().dfssm_conv_step(conv_state.data_ptr(), xbc.data_ptr(), xbc.stride(0),
-                                      conv_w.contiguous().data_ptr(), conv_b.contiguous().data_ptr(), B, C,
-                                      _C.stream()), "conv_step")
+    conv_w, conv_b = conv_w.contiguous(), conv_b.contiguous()
+    _C.check(_C.lib().dfssm_conv_step(conv_state.data_ptr(), xbc.data_ptr(), xbc.stride(0), conv_w.data_ptr(),
+                                      conv_b.data_ptr(), B, C, _C.stream()), "conv_step")
 
 
 def ssm_step(h: torch.Tensor, xbc: torch.Tensor, dt: torch.Tensor, dt_bias, A_log, D, y_out: torch.Tensor) -> None:
@@ -160,7 +163,7 @@ def ssm_step(h: torch.Tensor, xbc: torch.Tensor, dt: torch.Tensor, dt_bias, A_lo
     B, H, P, N = h.shape
     if not h.is_contiguous() or xbc.stride(1) != 1 or dt.stride(1) != 1 or y_out.stride(1) != 1:
         raise ValueError("h_state must be contiguous and xBC / dt / y_out rows contiguous")
+    dt_bias, A_log, D = dt_bias.contiguous(), A_log.contiguous(), D.contiguous()
     _C.check(_C.lib().dfssm_ssm_step(h.data_ptr(), xbc.data_ptr(), xbc.stride(0), dt.data_ptr(), dt.stride(0),
-                                     dt_bias.contiguous().data_ptr(), A_log.contiguous().data_ptr(),
-                                     D.contiguous().data_ptr(), y_out.data_ptr(), y_out.stride(0),
-                                     B, H, P, N, _C.stream()), "ssm_step")
+                                     dt_bias.data_ptr(), A_log.data_ptr(), D.data_ptr(), y_out.data_ptr(),
+                                     y_out.stride(0), B, H, P, N, _C.stream()), "ssm_step")

@@ -144,3 +144,51 @@ def test_silu_all_halves(w3):
     nan = np.isnan(rx)
     np.testing.assert_array_equal(np.isnan(got), nan)
     np.testing.assert_array_equal(got.view(np.uint16)[~nan], rx.view(np.uint16)[~nan])
+
+
+def _strided(a):
+    """The same values as every second element of a larger tensor."""
+    big = torch.zeros(*a.shape[:-1], 2 * a.shape[-1], dtype=a.dtype, device=a.device)
+    big[..., ::2] = a
+    return big[..., ::2]
+
+
+def test_strided_arguments():
+    """Several arguments that are not contiguous in one call: each operator's copies are all alive until its
+    launch, so no copy takes another's memory."""
+    rng = np.random.default_rng(31)
+    N, K, M = 256, 512, 2
+    packed = rng.integers(0, 1 << 32, (N, K // 32), dtype=np.uint32).view(np.int32)
+    bits = ops.tile_bits(torch.from_numpy(packed).to(DEV), N, K)
+    f = lambda *sh: _h(rng.uniform(0.5, 1.5, sh).astype(np.float16))
+    i8 = lambda *sh: torch.from_numpy(rng.integers(-127, 128, sh, dtype=np.int8)).to(DEV)
+    ws, q, xs, xn, lA, lAs, lBq = f(N), i8(M, K), f(M), f(M, K), i8(N, 16), f(N), f(16, K)
+    print("strided scaffold", flush=True)
+    ref = ops.scaffold_lora_gemm(bits, ws, q, xs, xn, lA, lAs, lBq, N)
+    got = ops.scaffold_lora_gemm(bits, *map(_strided, (ws, q, xs, xn, lA, lAs, lBq)), N)
+    for r, t in zip(ref, got):
+        assert torch.equal(r, t)
+
+    print("strided norm", flush=True)
+    x, w = f(M, K), torch.from_numpy(rng.uniform(0.5, 1.5, K).astype(np.float32)).to(DEV)
+    for r, t in zip(ops.rmsnorm_quantize(x, w), ops.rmsnorm_quantize(_strided(x), _strided(w))):
+        assert torch.equal(r, t)
+
+    print("strided conv", flush=True)
+    C = 512
+    cw, cb, st, xbc = f(C, 4), f(C), f(M, C, 3), f(M, C)
+    st2, xbc2 = st.clone(), xbc.clone()
+    ops.conv_step(st, xbc, cw, cb)
+    ops.conv_step(st2, xbc2, _strided(cw), _strided(cb))
+    assert torch.equal(st, st2) and torch.equal(xbc, xbc2)
+
+    print("strided ssm", flush=True)
+    H, P = 8, 16
+    h = torch.from_numpy(rng.normal(0, 1, (M, H, P, 128)).astype(np.float32)).to(DEV)
+    xbc, dt = f(M, H * P + 256), f(M, H)
+    v = [torch.from_numpy(rng.uniform(0.1, 2.0, H).astype(np.float32)).to(DEV) for _ in range(3)]
+    h2, y, y2 = h.clone(), torch.empty(M, H * P, dtype=torch.float16, device=DEV), None
+    y2 = torch.empty_like(y)
+    ops.ssm_step(h, xbc, dt, *v, y)
+    ops.ssm_step(h2, xbc, dt, *map(_strided, v), y2)
+    assert torch.equal(h, h2) and torch.equal(y, y2)
