@@ -70,7 +70,9 @@ def _stream_workspace(device, stream: int) -> torch.Tensor:
     dev = device if isinstance(device, torch.device) else torch.device(device)
     if torch.cuda.is_current_stream_capturing():
         return _new_scaffold_workspace(dev)
-    key = (dev.type, dev.index if dev.index is not None else torch.cuda.current_device(), stream)
+    if dev.index is None:
+        dev = torch.device(dev.type, torch.cuda.current_device())
+    key = (dev, stream)
     ws = _scaffold_ws.get(key)
     if ws is None:
         with _scaffold_ws_lock:
