@@ -130,7 +130,7 @@ def rmsnorm_quantize(x: torch.Tensor, w: torch.Tensor):
     _need(x, torch.float16, "x")
     _need(w, torch.float32, "w")
     M, K = x.shape
-    xn = torch.empty_like(x)
+    xn = torch.empty(M, K, dtype=torch.float16, device=x.device)
     q = torch.empty(M, K, dtype=torch.int8, device=x.device)
     s = torch.empty(M, dtype=torch.float16, device=x.device)
     x, w = x.contiguous(), w.contiguous()

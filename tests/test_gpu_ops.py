@@ -187,8 +187,17 @@ def test_strided_arguments():
     h = torch.from_numpy(rng.normal(0, 1, (M, H, P, 128)).astype(np.float32)).to(DEV)
     xbc, dt = f(M, H * P + 256), f(M, H)
     v = [torch.from_numpy(rng.uniform(0.1, 2.0, H).astype(np.float32)).to(DEV) for _ in range(3)]
-    h2, y, y2 = h.clone(), torch.empty(M, H * P, dtype=torch.float16, device=DEV), None
+    h2, y = h.clone(), torch.empty(M, H * P, dtype=torch.float16, device=DEV)
     y2 = torch.empty_like(y)
     ops.ssm_step(h, xbc, dt, *v, y)
     ops.ssm_step(h2, xbc, dt, *map(_strided, v), y2)
     assert torch.equal(h, h2) and torch.equal(y, y2)
+
+
+def test_rmsnorm_quantize_transposed_input():
+    """Rows that lie side by side in memory (a transposed tensor): the values of the row-major copy."""
+    x = _h(np.random.default_rng(32).normal(0, 1, (512, 3)).astype(np.float16)).t()
+    w = torch.ones(512, device=DEV)
+    print("transposed norm", flush=True)
+    for r, t in zip(ops.rmsnorm_quantize(x.contiguous(), w), ops.rmsnorm_quantize(x, w)):
+        assert torch.equal(r, t)
