@@ -232,21 +232,29 @@ def test_2p7b_layers_prefill_300_chunked():
 
 
 # ------------------------------------------------------------------------------ wide prefill vs the oracle
-@pytest.mark.parametrize("case", ["tiny_b16_t33", "2p7b_layers_b64_t6"])
+@pytest.mark.parametrize("case", ["tiny_b16_t33", "2p7b_layers_b64_t6", "d512_di5120_b64_t18", "d4608_di512_b64_t37"])
 def test_generate_wide_prefill_vs_oracle(case):
-    """generate(prompt=...) whose prefill takes the many-row kernels (prep_rows_kernel,
-    expand_bits_kernel, gemm_wide_kernel: one chunk of >= 256 rows), against the oracle's
-    step-by-step ingestion: greedy tokens and the logits of one more step identical, state within
-    1e-3. The tiny model at batch 16 with a 33-token prompt (512 prefill rows); config 4's layer
-    shapes with the full vocabulary at batch 64 with a 6-token prompt (320 rows)."""
+    """generate(prompt=...) whose prefill takes the many-row kernels (one chunk of more than 64 rows), against
+    the oracle's step-by-step ingestion: greedy tokens and the logits of one more step identical, state within
+    1e-3. Up to 1024 rows (prep_few_rows_kernel, the GEMM's narrow tile): the tiny model at batch 16 with a
+    33-token prompt (512 prefill rows); the 2.7B layer shapes with the full vocabulary at batch 64 with a
+    6-token prompt (320 rows). More (prep_rows_kernel): 1088 rows with the wide tile in in_proj, 2304 rows
+    with the wide tile in out_proj."""
     if case == "tiny_b16_t33":
         from dfssm.synth import config_tiny
         c, B, T, n = config_tiny(n_layer=3), 16, 33, 4
-    else:
+    elif case == "2p7b_layers_b64_t6":
         c = DFSSMConfig(n_layer=2, d_model=2560, d_inner=5120, d_state=128, nheads=80, headdim=64, ngroups=1,
                         vocab_size=50288, kw=4)
         B, T, n = 64, 6, 2
-    assert B * (T - 1) >= 256  # the wide path
+    else:
+        dm, di, T = (512, 5120, 18) if case.startswith("d512") else (4608, 512, 37)
+        c = DFSSMConfig(n_layer=1, d_model=dm, d_inner=di, d_state=128, nheads=di // 64, headdim=64, ngroups=1,
+                        vocab_size=1000, kw=4)
+        B, n = 64, 2
+        tiles = -(-B * (T - 1) // 64) * -(-(c.in_proj_out if dm == 512 else dm) // 256)
+        assert B * (T - 1) > 1024 and tiles >= 640  # 16 rows per prologue workgroup, the GEMM's wide tile
+    assert B * (T - 1) > 64  # the many-row kernels
     w = make_weights(c, seed=21)
     print(f"wide prefill vs oracle: {case}", flush=True)
     prompts = make_prompts(B, c.vocab_size, T, base_seed=4000)

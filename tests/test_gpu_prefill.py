@@ -107,13 +107,37 @@ def test_prefill_2p7b_layer_shapes():
     _prefill_vs_steps(w, 64, 20)
 
 
-@pytest.mark.parametrize("dm,di,B,T", [(1536, 3072, 5, 27), (1536, 3072, 5, 13), (512, 3584, 64, 19),
-                                        (4608, 512, 6, 43)])
-def test_prefill_many_rows(dm, di, B, T):
-    """The many-row prologue and GEMM (more than 64 rows) at odd multiples of 512 columns, one and two
-    passes of the LoRA contraction, row counts no tile divides, both widths of the GEMM's tile."""
-    c = DFSSMConfig(n_layer=2, d_model=dm, d_inner=di, d_state=128, nheads=di // 64, headdim=64, ngroups=1,
-                    vocab_size=1000, kw=4)
+def _many_row_forms(dm, di, rows):
+    """The forms that the many-row prologue (rows per workgroup, the same for both projections) and the wide GEMM
+    (outputs per workgroup, in_proj and out_proj) take at a chunk of `rows` rows: the rules of launch_prep and
+    launch_gemm_wide_mode."""
+    assert rows > 64
+    wide = lambda n: 256 if -(-rows // 64) * -(-n // 256) >= 640 else 128
+    return 4 if rows <= 1024 else 16, wide(2 * di + 2 * 128 + di // 64), wide(dm)
+
+
+@pytest.mark.parametrize("dm,di,B,T,forms", [
+    # up to 1024 rows: four rows per workgroup of the prologue
+    (1536, 3072, 5, 27, (4, 128, 128)),
+    (1536, 3072, 5, 13, (4, 128, 128)),      # 65 rows: the smallest chunk of these kernels
+    (4608, 512, 6, 43, (4, 128, 128)),
+    (512, 512, 64, 16, (4, 128, 128)),       # 1024 rows
+    # more: 16 rows per workgroup
+    (2048, 4096, 5, 205, (16, 128, 128)),    # 1025 rows: one live row in the last workgroup; the 1.3B shape
+    (512, 3584, 64, 19, (16, 128, 128)),
+    (1536, 3072, 33, 33, (16, 128, 128)),    # 1089 rows; the LoRA contraction in one pass (3) and in two (6)
+    # the wide tile of the GEMM, rows that no tile divides
+    (2048, 4096, 37, 33, (16, 256, 128)),    # 1221 rows
+    (4608, 512, 33, 69, (16, 128, 256)),     # 2277 rows: 648 tiles of out_proj
+    (2560, 5120, 63, 65, (16, 256, 256)),    # 4095 rows: the 2.7B shape in the forms of its largest chunks
+])
+def test_prefill_many_rows(dm, di, B, T, forms):
+    """The many-row prologue and GEMM (more than 64 rows) in each of their forms: both row counts of the
+    prologue's workgroups and both sides of the switch, both widths of the GEMM's tile in both projections, odd
+    multiples of 512 columns, one and two passes of the LoRA contraction, row counts that neither divides."""
+    assert _many_row_forms(dm, di, B * T) == forms
+    c = DFSSMConfig(n_layer=2 if dm < 2048 else 1, d_model=dm, d_inner=di, d_state=128, nheads=di // 64, headdim=64,
+                    ngroups=1, vocab_size=1000, kw=4)
     print(f"prefill rows {B * T} of {dm} / {di}", flush=True)
     _prefill_vs_steps(make_weights(c, seed=11), B, T)
 
