@@ -146,6 +146,62 @@ def test_silu_all_halves(w3):
     np.testing.assert_array_equal(got.view(np.uint16)[~nan], rx.view(np.uint16)[~nan])
 
 
+def _silu_inputs():
+    """fp32 values o for the kernels' o sigmoid(o): every float within 2000 steps of the ends of its exponential's
+    range; the floats within two steps of each point where o sigmoid(o) changes its fp16 rounding, on each of its
+    three monotonic branches; and values spread over the logarithm of [2^-14, 104]."""
+    ends = np.array([86.0, 87.0, 88.0, 88.72284, 89.0, 103.97], np.float32).view(np.int32)
+    edge = (ends[:, None] + np.arange(-2000, 2001)[None]).astype(np.int32).view(np.float32).ravel()
+    halves = np.arange(1, 31743, dtype=np.uint16).view(np.float16).astype(np.float64)
+    mid = (halves[:-1] + halves[1:]) / 2
+    bottom = -1.2784645427610738  # the minimum of o sigmoid(o), -0.27846
+    points = []
+    for lo, hi, v in ((0.0, 66000.0, mid), (bottom, 0.0, -mid[mid < 0.2784]), (-30.0, bottom, -mid[mid < 0.2784])):
+        lo, hi = np.full_like(v, lo), np.full_like(v, hi)
+        rising = hi[0] > bottom
+        for _ in range(60):
+            c = (lo + hi) / 2
+            below = c / (1 + np.exp(-c)) < v
+            lo, hi = np.where(below == rising, c, lo), np.where(below == rising, hi, c)
+        points.append(lo[np.abs(lo) >= 2.0 ** -14])
+    p = np.concatenate(points).astype(np.float32).view(np.int32)
+    near = (p[:, None] + np.arange(-2, 3)[None]).astype(np.int32).view(np.float32).ravel()
+    rng = np.random.default_rng(33)
+    spread = np.exp(rng.uniform(np.log(2.0 ** -14), np.log(104.0), 400000)).astype(np.float32)
+    return np.concatenate([edge, -edge, near, spread, -spread])
+
+
+def test_silu_sweep():
+    """SiLU at fp32 inputs, where the clamps and roundings of the kernels' sigmoid could show (the conv feeds it
+    fp32 sums), against the oracle's formula, bit for bit. Each input is the exact sum of three taps: the
+    bytes of its 24-bit integer times powers of two."""
+    o = _silu_inputs()
+    m, e = np.frexp(np.abs(o).astype(np.float64))
+    m = (m * 2 ** 24).astype(np.int64)
+    e = e - 24  # |o| = m 2^e
+    taps, weights = [], []
+    for sh in (16, 8, 0):
+        t = e + sh
+        k = np.clip(t, -24, 15)  # the weight's exponent; the rest goes to the byte
+        taps.append(np.ldexp(((m >> sh) & 255).astype(np.float64) * np.sign(o), t - k).astype(np.float16))
+        weights.append(np.ldexp(1.0, k).astype(np.float16))
+    total = sum(a.astype(np.float64) * b.astype(np.float64) for a, b in zip(taps, weights))
+    np.testing.assert_array_equal(total, o.astype(np.float64))
+    C = o.size
+    w = np.zeros((C, 4), np.float16)
+    st = np.zeros((1, C, 3), np.float16)
+    for i in range(2):
+        st[0, :, 1 + i], w[:, 1 + i] = taps[i], weights[i]
+    w[:, 3] = weights[2]
+    x, b = taps[2].reshape(1, C), np.zeros(C, np.float16)
+    print(f"silu at {C} fp32 inputs", flush=True)
+    gx = _h(x)
+    ops.conv_step(_h(st), gx, _h(w), _h(b))
+    rx = np.ascontiguousarray(x)
+    O.conv_step(st.copy(), rx, w, b)
+    np.testing.assert_array_equal(_np16(gx).view(np.uint16), rx.view(np.uint16))
+
+
 def _strided(a):
     """The same values as every second element of a larger tensor."""
     big = torch.zeros(*a.shape[:-1], 2 * a.shape[-1], dtype=a.dtype, device=a.device)

@@ -12,6 +12,7 @@ import pytest
 import torch
 
 from df_ssm_inference import DFSSMModel
+from dfssm import _C
 from dfssm.format import DFSSMConfig
 from dfssm.synth import config_1p3b, config_tiny, make_prompts, make_weights
 from oracle import oracle as O
@@ -183,3 +184,69 @@ def test_prefill_readout_order(B, T, heads, headdim):
     st.ingest(prompts[:, :-1], step_by_step=True)
     ls = st.forward(prompts[:, -1].to(DEV))
     _assert_same(pf, st, lp, ls)
+
+
+def _gate_weights(z):
+    """A one-layer model whose gate gets the halves z in every row and whose SSM readout is 1: the embedding is
+    all ones, LoRA ranks 0 and 1 of in_proj carry 16 and 1, so that an integer 16 a + b times a power of two,
+    any fp16 value, comes from the int8 factors a and b and the row scale; no scaffold term; x = silu of the
+    conv bias, B = C = 0 and D = 1 / x."""
+    c = DFSSMConfig(n_layer=1, d_model=512, d_inner=z.size, d_state=128, nheads=z.size // 64, headdim=64, ngroups=1,
+                    vocab_size=1000, kw=4)
+    w = make_weights(c, seed=1)
+    w.emb[:], w.emb_scale[:] = 1, 1
+    L = w.layers[0]
+    L["ln_w"][:] = 1
+    L["in_scale"][:] = 0
+    L["in_lB"][:], L["in_lB_s"][:] = 0, 1
+    L["in_lB"][0, 0], L["in_lB"][1, 0] = 16, 1
+    m, e = np.frexp(z.astype(np.float64))
+    e = np.maximum(e - 11, -24)  # z = m 2^e with |m| < 2048
+    inf, nan = np.isinf(z), np.isnan(z)
+    m = np.ldexp(np.where(inf | nan, 0, z.astype(np.float64)), -e).astype(np.int64)
+    a, b, s = np.abs(m) // 16 * np.sign(m), np.abs(m) % 16 * np.sign(m), np.ldexp(1.0, e)
+    a = np.where(inf, np.where(z > 0, 127, -127), np.where(nan, 127, a))
+    b, s = np.where(nan, -127, b), np.where(inf | nan, 65504.0, s)  # inf - inf
+    L["in_lA"][:], L["in_lA_s"][:] = 0, 1
+    L["in_lA"][:z.size, 0], L["in_lA"][:z.size, 1], L["in_lA_s"][:z.size] = a, b, s
+    L["conv_w"][:] = 0
+    L["conv_b"][:z.size], L["conv_b"][z.size:] = 2, 0
+    x = np.zeros((1, 1), np.float16)
+    O.conv_step(np.zeros((1, 1, 3), np.float16), x, np.zeros((1, 4), np.float16), np.full(1, 2, np.float16))
+    L["D"][:] = 1 / np.float32(x[0, 0])
+    return w
+
+
+def test_gate_all_halves():
+    """The gate fp16(z fp16(sigmoid(z))) of every fp16 z but -0 (all finite values, the infinities, one NaN) in the
+    batched decode step and in the prefill scan, as both leave it in their workspaces' g rows, against the
+    oracle's formula, bit for bit."""
+    bits = np.concatenate([np.arange(0, 0x7c02), np.arange(0x8001, 0xfc01)]).astype(np.uint16)
+    B, DI = 5, 5120
+    n = -(-bits.size // DI)
+    bits = np.concatenate([bits, np.zeros(n * DI - bits.size, np.uint16)]).reshape(n, DI)
+    align = lambda v: -(-v // 256) * 256
+    for i in range(n):
+        z = bits[i].view(np.float16)
+        ref = O.gate(np.ones((1, DI), np.float16), z.reshape(1, DI))[0]
+        w = _gate_weights(z)
+        gpu = DFSSMModel.from_weights(w, device=DEV, batch_size=B)
+        ld = w.cfg.in_proj_out
+        print(f"gate of halves {i + 1} / {n}", flush=True)
+        gpu.prefill(torch.zeros(B, 1, dtype=torch.int64))
+        proj = align(B * w.cfg.d_model * 2)                      # rows of x, then of in_proj, then of g
+        pf = gpu._pf_ws[proj:].view(torch.float16)[:B * ld].view(B, ld)[:, :DI].cpu().numpy()
+        nan = np.isnan(z)
+        np.testing.assert_array_equal(pf[0].view(np.uint16)[~nan], z.view(np.uint16)[~nan])  # the gate's input
+        rows = [gpu._pf_ws[proj + align(B * ld * 2):]]
+        x = torch.ones(B, w.cfg.d_model, dtype=torch.float16, device=DEV)
+        gpu.reset_state()
+        for ph in range(3):  # in_proj's prologue, in_proj + conv, SSM + gate
+            _C.check(_C.lib().dfssm_layer_phase(gpu._model, 0, ph, x.data_ptr(), gpu._state, gpu.workspace.data_ptr(),
+                                                _C.stream()))
+        rows.append(gpu.workspace[align(B * ld * 2):])           # rows of in_proj, then of g
+        for r in rows:
+            got = r.view(torch.float16)[:B * DI].view(B, DI).cpu().numpy()
+            assert np.isnan(got[:, nan]).all()
+            for b in range(B):
+                np.testing.assert_array_equal(got[b].view(np.uint16)[~nan], ref.view(np.uint16)[~nan])
