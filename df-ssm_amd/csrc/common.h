@@ -168,6 +168,28 @@ __device__ __forceinline__ double wave_sum_dpp_f64(double v) {
   v = row_sum_f64(v);
   return (readlane_f64(v, 0) + readlane_f64(v, 16)) + (readlane_f64(v, 32) + readlane_f64(v, 48));
 }
+// wave_sum_dpp_f64 of four values at once, added up in order: (((ss + sum a) + sum b) + sum c) + sum d, in 45
+// instructions instead of 96. After the two steps within the quads lane 4 i + k holds the quad's sum of value k
+// (each lane sends the value its partner keeps), and the rest of the tree keeps the lane's place in its quad.
+__device__ __forceinline__ double wave_sums4_dpp_f64(double ss, double a, double b, double c, double d) {
+  const bool odd = threadIdx.x & 1, hi = threadIdx.x & 2;
+  const double u = (odd ? b : a) + dpp_f64<0xB1>(odd ? a : b);
+  const double w = (odd ? d : c) + dpp_f64<0xB1>(odd ? c : d);
+  double v = (hi ? w : u) + dpp_f64<0x4E>(hi ? u : w);
+  v += dpp_f64<0x124>(v);
+  v += dpp_f64<0x128>(v);
+  uint64_t x = __builtin_bit_cast(uint64_t, v);  // rows 0 + 1, 2 + 3, then the halves
+  auto l = __builtin_amdgcn_permlane16_swap((uint32_t)x, (uint32_t)x, false, false);
+  auto h = __builtin_amdgcn_permlane16_swap((uint32_t)(x >> 32), (uint32_t)(x >> 32), false, false);
+  v = __builtin_bit_cast(double, ((uint64_t)h[0] << 32) | l[0]) + __builtin_bit_cast(double, ((uint64_t)h[1] << 32) | l[1]);
+  x = __builtin_bit_cast(uint64_t, v);
+  l = __builtin_amdgcn_permlane32_swap((uint32_t)x, (uint32_t)x, false, false);
+  h = __builtin_amdgcn_permlane32_swap((uint32_t)(x >> 32), (uint32_t)(x >> 32), false, false);
+  v = __builtin_bit_cast(double, ((uint64_t)h[0] << 32) | l[0]) + __builtin_bit_cast(double, ((uint64_t)h[1] << 32) | l[1]);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) ss += readlane_f64(v, k);
+  return ss;
+}
 __device__ __forceinline__ int wave_sum_dpp_i32(int v) {
   v += dpp_i32<0xB1>(v);
   v += dpp_i32<0x4E>(v);
@@ -198,8 +220,8 @@ __device__ __forceinline__ void lds_barrier() {
 }
 
 // Block-wide sums / max for blockDim.x == NT (multiple of 64). `red` must hold NT/64 entries.
-// Every sum reduced this way in the decode kernels is exact (fp64 sums of exactly representable
-// products, integer sums), so the reduction order does not change results.
+// The sums reduced this way are of integers or of exactly representable products in fp64, where two orders
+// are a few units of 2^-53 apart at most.
 template <int NT>
 __device__ __forceinline__ double block_sum_f64(double v, double* red) {
   v = wave_sum_dpp_f64(v);

@@ -47,7 +47,9 @@
 //
 // Arithmetic is that of prep_kernel + proj_kernel + ssm_kernel; every sum that the kernels
 // split differently (sum of squares, LoRA intermediate and LoRA term, C.h readout) is a sum of
-// exactly representable products accumulated in fp64, and integer sums are exact.
+// exactly representable products accumulated in fp64, where two orders are a few units of 2^-53
+// apart at most and round to the same fp32 value unless a boundary lies between them; integer sums
+// are exact.
 #include "common.h"
 #include "dfssm_kernels.h"
 

@@ -112,7 +112,7 @@ __device__ __forceinline__ void gemm_in_prologue(const GemmPro& p, int D, int m,
     part += x0 * x0;
     part += x1 * x1;
   }
-  {  // sum of squares (fp64: the sums are exact)
+  {  // sum of squares
     const double pw = wave_sum_dpp_f64(part);
     if (lane == 0) pr_d[w] = pw;
   }

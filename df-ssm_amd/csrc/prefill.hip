@@ -10,10 +10,14 @@
 //                    blocks): the fp32 state stays in registers for all n tokens (read and written
 //                    once per layer instead of once per token).
 //
-// Every rounding and every sum whose order could show is the decode step's (ssm_kernel), so
-// together with the row-wise kernels the prefill equals, bit for bit, n calls of the decode step
-// (Mamba-2 recurrence of df_ssm_kernels.cu:53-103 / training/df_ssm_mamba2_distill_dfw.py:346-381,
-// evaluated token by token as the reference's cpu_inference_driver.py:186-204 ingests a prompt).
+// Every rounding here and the order of the scan's readout are the decode step's (ssm_kernel), so together
+// with the row-wise kernels the prefill equals n calls of the decode step bit for bit (Mamba-2
+// recurrence of df_ssm_kernels.cu:53-103 / training/df_ssm_mamba2_distill_dfw.py:346-381, evaluated
+// token by token as the reference's cpu_inference_driver.py:186-204 ingests a prompt), up to the fp64
+// sums that the decode's launches and the prefill add in different orders: sum(x^2) and sum(g^2) (here in
+// prep_kernel's order at every row count) and the LoRA sums (above 64 rows on the fp64 matrix cores). Two
+// orders are a few units of 2^-53 apart at most, which shows only where an fp32 rounding boundary lies
+// between them: about one row in 10^9 for sum(g^2).
 #include <type_traits>
 
 #include "common.h"

@@ -88,7 +88,7 @@ __global__ __launch_bounds__(kPT) void prep_kernel(PrepArgs a, int M) {
   } else {
     part = tid < a.n_slots ? slot : 0.0;
   }
-  {  // sum of squares (fp64: the sums are exact)
+  {  // sum of squares
     const double pw = wave_sum_dpp_f64(part);
     if (lane == 0) L.red_d[w] = pw;
   }
@@ -203,6 +203,10 @@ __global__ __launch_bounds__(kPT) void prep_kernel(PrepArgs a, int M) {
 // both come as 16-byte vectors. The 16 rows of q are one contiguous block of the wide GEMM's layout
 // (kWideTile): staged in LDS (the rows of the 16-byte units swizzled by step and group, which are
 // multiples of 256 bytes apart) and stored as one, the rows past M with copies of the last one.
+// The squares are added in prep_kernel's order, one wave sum per 512 columns: more than a third of the sums over
+// gated rows are not exact in fp64, and a row's norm must not depend on how many rows a chunk has. (Against one
+// wave sum per row that costs 0.3% of the call at 1056 rows of the 1.3B shape; 0.7% without the four
+// sums per butterfly.)
 //
 // What bounds it: VALU issue (about 18 instructions per value) and the fp64 matrix rate, both about
 // 9 us per workgroup at K = 5120, one workgroup per CU. Measured against one workgroup of K / 8 threads
@@ -229,15 +233,21 @@ __global__ __launch_bounds__(kPrepRowsT) void prep_rows_kernel(PrepArgs a, int M
   u32x4 v[KB];
 #pragma unroll
   for (int j = 0; j < KB; ++j) v[j] = *(const u32x4*)(act + 512 * j);
-  double part = 0.0;
+  double part[KB], ss = 0.0;  // added in prep_kernel's order: its wave j holds the 512 columns of chunk j
 #pragma unroll
-  for (int j = 0; j < KB; ++j)
+  for (int j = 0; j < KB; ++j) {
+    part[j] = 0.0;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const double x = (double)h2f((uint16_t)(v[j][e >> 1] >> (16 * (e & 1))));
-      part = __builtin_fma(x, x, part);  // (x x is exact)
+      part[j] = __builtin_fma(x, x, part[j]);  // (x x is exact)
     }
-  const float var = (float)wave_sum_dpp_f64(part) * (1.0f / (float)K);
+  }
+#pragma unroll
+  for (int j = 0; j + 4 <= KB; j += 4) ss = wave_sums4_dpp_f64(ss, part[j], part[j + 1], part[j + 2], part[j + 3]);
+#pragma unroll
+  for (int j = KB & ~3; j < KB; ++j) ss += wave_sum_dpp_f64(part[j]);
+  const float var = (float)ss * (1.0f / (float)K);
   const float r = 1.0f / sqrt_rn(var + 1e-5f);
   float mx = 0.0f;
 #pragma unroll
@@ -333,13 +343,13 @@ __global__ __launch_bounds__(kPrepRowsT) void prep_rows_kernel(PrepArgs a, int M
 // turn, two exchanges through LDS), and the LoRA contraction of 4 rows x 16 ranks runs on
 // v_mfma_f64_4x4x4_4b (the four blocks are four ranks each on the same rows), whose rate is the 16 x 16
 // instruction's at a quarter of the rows; q goes straight to its place, 64 contiguous bytes per step and
-// group.
+// group. The squares are added in prep_kernel's order here as well.
 template <int KB>
 __global__ __launch_bounds__(kPrepRowsT) void prep_few_rows_kernel(PrepArgs a, int M) {
   constexpr int K = 512 * KB, KW = (KB + 3) / 4;  // chunks per wave at most
   constexpr int XS = 2 * K + 16;                  // LDS bytes of a row of xn (padded)
   __shared__ __attribute__((aligned(16))) uint8_t xn[4 * XS];
-  __shared__ double red_d[16], part_h[16][64];
+  __shared__ double red_d[4][KB], part_h[16][64];
   __shared__ float red_f[16];
   __shared__ int red_i[16];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -357,20 +367,22 @@ __global__ __launch_bounds__(kPrepRowsT) void prep_few_rows_kernel(PrepArgs a, i
 #pragma unroll
   for (int j = 0; j < KB; ++j) bv[j] = *(const u32x4*)(a.lBq + (size_t)li * K + 512 * j + 32 * w + 8 * g);
   asm volatile("" ::: "memory");  // issued here, not sunk to their use
-  double part = 0.0;
 #pragma unroll
   for (int i = 0; i < KW; ++i) {
     if (qd + 4 * i >= KB) break;
+    double part = 0.0;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const double x = (double)h2f((uint16_t)(v[i][e >> 1] >> (16 * (e & 1))));
       part = __builtin_fma(x, x, part);  // (x x is exact)
     }
+    part = wave_sum_dpp_f64(part);
+    if (lane == 0) red_d[r4][qd + 4 * i] = part;
   }
-  part = wave_sum_dpp_f64(part);
-  if (lane == 0) red_d[w] = part;
   lds_barrier();
-  const double ss = (red_d[r4] + red_d[r4 + 4]) + (red_d[r4 + 8] + red_d[r4 + 12]);
+  double ss = 0.0;  // prep_kernel's order: its wave j holds the 512 columns of chunk j
+#pragma unroll
+  for (int j = 0; j < KB; ++j) ss += red_d[r4][j];
   const float r = 1.0f / sqrt_rn((float)ss * (1.0f / (float)K) + 1e-5f);
   float mx = 0.0f;
 #pragma unroll

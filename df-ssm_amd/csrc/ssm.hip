@@ -126,7 +126,7 @@ __global__ __launch_bounds__(256) void ssm_kernel(SsmArgs a) {
 // blocks of sequence 0, of sequence 1, ..., then 16 prologue workgroups per sequence (one per
 // LoRA rank r): each polls the whole row of g from the tagged words, computes the gated RMSNorm
 // (sum of g^2 from g itself), the maximum, the scale and rank r's intermediate, and writes the q
-// bytes of column slice r. Every sum is a sum of exact products in fp64 (prep_kernel's values).
+// bytes of column slice r. Every sum is a sum of exact products in fp64 (prep_kernel's, in another order).
 // Tags: every workgroup keeps its own launch count (read at the start, written back at the end);
 // all of them start at zero and every launch runs every workgroup once, so all workgroups of a
 // launch derive the same tag, and a word of the previous launch carries another one.
@@ -206,7 +206,7 @@ __device__ __forceinline__ void gated_prologue(const SsmPrepArgs& a, int rr, int
     part += g0 * g0;
     part += g1 * g1;
   }
-  {  // sum of squares (fp64: the sums are exact)
+  {  // sum of squares
     const double pw = wave_sum_dpp_f64(part);
     if (lane == 0) red_d[w] = pw;
   }

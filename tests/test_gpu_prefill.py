@@ -186,6 +186,62 @@ def test_prefill_readout_order(B, T, heads, headdim):
     _assert_same(pf, st, lp, ls)
 
 
+def _norm_order_weights(chunk, small):
+    """A one-layer model whose tokens all embed to one row of 2560 columns with a sum of squares that rounds to fp32
+    one way or the other by the order of its fp64 sum. The large columns (2^15 and 8, the first two of a
+    512-column chunk; n of 32) make 2^30 + 64 + 1024 n, in the middle of two fp32 values; the small ones (2^-12)
+    count only if at least 2^-22 of their squares is added up before it meets the 2^30. The norm weights put
+    the normalized values of the n columns where the two results round to different halves."""
+    K, f4 = 2560, np.float32
+    x = np.zeros(K, np.float16)
+    x[512 * chunk:512 * chunk + 2] = 2.0 ** 15, 8.0
+    assert not x[small].any()
+    x[small] = 2.0 ** -12
+
+    def scale(ss):  # 1 / sqrt(ss / K + 1e-5) as the kernels round it
+        var = f4(f4(ss) * (f4(1) / f4(K)))
+        return f4(1) / np.sqrt(var + f4(1e-5))
+
+    for n in range(200, 400):
+        lost = 2.0 ** 30 + 64 + 1024 * n
+        r0, r1 = scale(lost), scale(lost + 2.0 ** -22)
+        if r0 != r1:
+            break
+    assert r0 != r1 and lost + 2.0 ** -23 == lost
+    fill = np.arange(600, 600 + n)
+    x[fill] = 32.0
+    w = np.ones(K, f4)
+    w[512 * chunk] = 0.01
+    halves = np.arange(0x3c00, 0x3c00 + n, dtype=np.uint16).view(np.float16).astype(np.float64)
+    near = ((halves + 2.0 ** -11) / (32.0 * float(r0))).astype(f4).view(np.int32)
+    w[fill] = near.view(f4)
+    for d in range(-8, 9):  # the weight's last bits
+        c = (near + d).astype(np.int32).view(f4)
+        differ = ((f4(32) * r0) * c).astype(np.float16) != ((f4(32) * r1) * c).astype(np.float16)
+        w[fill[differ]] = c[differ]
+    flips = (((f4(32) * r0) * w[fill]).astype(np.float16) != ((f4(32) * r1) * w[fill]).astype(np.float16)).sum()
+    assert flips > n // 2
+    c = DFSSMConfig(n_layer=1, d_model=K, d_inner=512, d_state=128, nheads=8, headdim=64, ngroups=1, vocab_size=1000,
+                    kw=4, emb_code=0)
+    wt = make_weights(c, seed=2)
+    wt.emb[:] = x
+    wt.layers[0]["ln_w"][:] = w
+    return wt
+
+
+@pytest.mark.parametrize("chunk,lanes", [(0, None), (0, (2, 3)), (0, (1, 2)), (3, (4, 8)), (3, (8, 12)), (3, (16, 32)),
+                                         (4, (32, 48))])
+def test_prefill_norm_order(chunk, lanes):
+    """The prefill's prologue adds its squares in the order of the decode step's (prep_kernel) in each of its forms:
+    60, 65 and 1025 rows. The small columns lie 2048 columns behind the large one (None), or two each in two
+    lanes of its chunk (8 columns a lane), which the tree adds to each other first or to the large one."""
+    small = np.arange(2048, 2056) if lanes is None else np.concatenate([512 * chunk + 8 * l + np.arange(2, 4) for l in lanes])
+    w = _norm_order_weights(chunk, small)
+    for B, T in ((5, 12), (5, 13), (5, 205)):
+        print(f"norm order chunk {chunk} lanes {lanes} B={B} T={T}", flush=True)
+        _prefill_vs_steps(w, B, T)
+
+
 def _gate_weights(z):
     """A one-layer model whose gate gets the halves z in every row and whose SSM readout is 1: the embedding is
     all ones, LoRA ranks 0 and 1 of in_proj carry 16 and 1, so that an integer 16 a + b times a power of two,
