@@ -76,8 +76,8 @@ WsLayout ws_layout(const dfssm_dims* d) {
 }
 
 // Prompt prefill workspace for up to `rows` = batch x tokens-per-chunk activation rows: the
-// residual stream of every row, the projection rows, g, the sum(g^2) slots and the prologue
-// outputs (q, scale, LoRA intermediate).
+// residual stream of every row, the projection rows, g (x before the scan), B | C after the conv, the
+// decay factors and the prologue outputs (q, its row sums, scale, LoRA intermediate).
 struct PfLayout {
   size_t x, proj, g, bc, dec, q, qs, xs, h, total;
 };
@@ -95,7 +95,7 @@ PfLayout pf_layout(const Derived& r, int rows) {
   w.g = off;     off = align_up(off + (size_t)rows * r.DI * 2);
   w.bc = off;    off = align_up(off + (size_t)rows * 2 * r.N * 2);
   w.dec = off;   off = align_up(off + (size_t)rows * r.H * 8);
-  w.q = off;     off = align_up(off + (size_t)(rows + 15) / 16 * 16 * kq);  // rows padded to 16 (tiled)
+  w.q = off;     off = align_up(off + (size_t)(rows + kWideTile - 1) / kWideTile * kWideTile * kq);
   w.qs = off;    off = align_up(off + (size_t)rows * 4);
   w.xs = off;    off = align_up(off + (size_t)rows * 4);
   w.h = off;     off = align_up(off + (size_t)rows * 16 * 4);

@@ -112,8 +112,9 @@ __device__ __forceinline__ void argmax_pairs(const HeadArgs& a, int M, int NG, i
 
 // x_next[m] = the embedding of token toks[m], m < M, by NT threads in 16-byte table chunks (16
 // int8 or 8 fp16 values), KB chunks per thread loaded before any is converted and stored.
-template <bool F16, int NT, int KB = 8>
+template <bool F16, int NT>
 __device__ __forceinline__ void embed_next(const HeadArgs& a, const int* toks, int M, int D) {
+  constexpr int KB = 8;
   const int CH = F16 ? D / 8 : D / 16, n = M * CH;
   for (int c0 = (int)threadIdx.x; c0 < n; c0 += NT * KB) {
     u32x4 ch[KB];

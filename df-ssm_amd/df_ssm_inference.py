@@ -457,11 +457,11 @@ class DFSSMModel:
             self._gen_graphs[S] = (self._capture(body), hist)
         return self._gen_graphs[S]
 
-    PREFILL_MAX_ROWS = 16384  # batch x tokens per prefill chunk (workspace ~ rows x 38 KB at 1.3B)
+    PREFILL_MAX_ROWS = 16384  # batch x tokens per prefill chunk (workspace ~ rows x 34.5 KB at 1.3B)
 
     def prefill(self, prompt: torch.Tensor, want_logits: bool = False) -> torch.Tensor:
         """Consume a (batch, T) prompt in one layer-major pass (dfssm_prefill): bit-for-bit the
-        result of T decode steps. Afterwards self._next holds the greedy token after the prompt
+        result of T decode steps (but for fp64 sums added in another order, see include/dfssm.h). Afterwards self._next holds the greedy token after the prompt
         and self.x its embedding; returns the last token's logits if want_logits, else None."""
         prompt = torch.as_tensor(prompt)
         if prompt.dim() == 1:

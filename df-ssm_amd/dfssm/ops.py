@@ -68,7 +68,7 @@ def scaffold_workspace(device) -> torch.Tensor:
 
 def _stream_workspace(device, stream: int) -> torch.Tensor:
     dev = device if isinstance(device, torch.device) else torch.device(device)
-    if torch.cuda.is_current_stream_capturing():
+    if stream and torch.cuda.is_current_stream_capturing():  # (the null stream cannot be captured)
         return _new_scaffold_workspace(dev)
     if dev.index is None:
         dev = torch.device(dev.type, torch.cuda.current_device())

@@ -289,7 +289,9 @@ size_t dfssm_prefill_workspace_bytes(const dfssm_dims* dims, int max_rows);
  * prompt rows of all sequences go through a layer together (prologues and scaffold GEMMs over
  * batch x n_tokens rows on the int8 matrix cores), the conv and the SSM recurrence walk the
  * tokens with their state in registers, so weights and state are read once per layer and chunk
- * instead of once per token. The prompt is processed in chunks of max_rows / batch tokens;
+ * instead of once per token. (Bit-for-bit up to the fp64 sums of squares and of the LoRA term that the
+ * two add in different orders: a few units of 2^-53, which reach a result where an fp32 rounding boundary
+ * lies between them, about one row in 10^9.) The prompt is processed in chunks of max_rows / batch tokens;
  * prefill_workspace holds dfssm_prefill_workspace_bytes(dims, max_rows) bytes, workspace is the
  * decode workspace (the head and the error flag). logits (batch, V) may be NULL; x receives the
  * embedding of `next` if fuse_next_embed, else the last token's residual row. */
