@@ -106,6 +106,20 @@ def test_scaffold_lora_op_shared_workspace():
     assert (counts == one_launch).all()  # every workgroup index counted every one-launch call
 
 
+def test_scaffold_lora_op_tags_wrap():
+    """The 16-bit tag of a call's words comes round after 65 536 calls: a call of four rows with the tag of an
+    earlier one, calls of one row between them (the counts are set forward in place of most of these, but not
+    past one that 2^14 divides), waits for its own words."""
+    wsx = torch.zeros(ops.SCAFFOLD_WORKSPACE_BYTES // 4, dtype=torch.int32, device=DEV)
+    for i, (M, count) in enumerate([(4, 5), (1, 16384), (1, 65540), (4, 65541), (2, 81920), (3, 131077),
+                                          (2, 147456), (4, 196613)]):
+        print(f"tag wrap: call {count + 1} with {M} rows", flush=True)
+        wsx[:256] = count
+        args, ref = _lora_op_case(8512, 2048, M, 30 + i)
+        _check_lora_op(ops.scaffold_lora_gemm(*args, workspace=wsx), ref)
+    assert ops.scaffold_error(wsx) == 0
+
+
 def test_scaffold_lora_op_streams_and_graphs():
     """Calls with the automatic workspace on two streams that may overlap, and in a captured graph replayed
     between eager calls: every result is the oracle's."""
