@@ -210,8 +210,8 @@ __global__ __launch_bounds__(kPT) void prep_kernel(PrepArgs a, int M) {
 //
 // What bounds it: VALU issue (about 18 instructions per value) and the fp64 matrix rate, both about
 // 9 us per workgroup at K = 5120, one workgroup per CU. Measured against one workgroup of K / 8 threads
-// walking 16 rows one after the other (a row's 16 ranks as fp64 fmas and wave reductions): 497 -> 123
-// us at 16 384 rows of K = 5120, 337 -> 65 us at K = 2560, 89 -> 22 and 67 -> 13 us at 999 rows of K =
+// walking 16 rows one after the other (a row's 16 ranks as fp64 fmas and wave reductions): 497 -> 124
+// us at 16 384 rows of K = 5120, 337 -> 66 us at K = 2560, 89 -> 22 and 67 -> 13 us at 999 rows of K =
 // 4096 and 2048 (63 workgroups: one round).
 // ------------------------------------------------------------------------------------------
 constexpr int kPrepRowsT = 1024;
