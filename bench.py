@@ -342,7 +342,7 @@ def scaffold_op_bytes(M, N, K):
 
 
 def scaffold_microbench(Ms=(1, 4, 16, 32), min_bytes=1 << 30, reps=3):
-    """BASELINE config 1 in isolation: in_proj (K 2048 -> N 8512) and out_proj (K 4096 -> N 2048),
+    """The scaffold operator in isolation: in_proj (K 2048 -> N 8512) and out_proj (K 4096 -> N 2048),
     each call = dfssm_scaffold_lora_gemm (LoRA intermediates + scaffold GEMV/GEMM + LoRA epilogue).
     The calls rotate over distinct weight copies (bits, scales, LoRA A, LoRA-B table) totalling more
     than `min_bytes`, so the weights stream from HBM, not from the 256 MB last-level cache; one graph

@@ -205,8 +205,8 @@ __global__ __launch_bounds__(kPT) void prep_kernel(PrepArgs a, int M) {
 // multiples of 256 bytes apart) and stored as one, the rows past M with copies of the last one.
 // The squares are added in prep_kernel's order, one wave sum per 512 columns: more than a third of the sums over
 // gated rows are not exact in fp64, and a row's norm must not depend on how many rows a chunk has. (Against one
-// wave sum per row that costs 0.3% of the call at 1056 rows of the 1.3B shape; 0.7% without the four
-// sums per butterfly.)
+// wave sum per row that costs 0.3 to 0.6% of the call at 1056 rows of the 1.3B shape, 0.1 to 0.3% at 16 384 of
+// the 2.7B; the first was 0.7% without the four sums per butterfly.)
 //
 // What bounds it: VALU issue (about 18 instructions per value) and the fp64 matrix rate, both about
 // 9 us per workgroup at K = 5120, one workgroup per CU. Measured against one workgroup of K / 8 threads

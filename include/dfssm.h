@@ -299,7 +299,7 @@ int dfssm_prefill(const dfssm_model* model, const int64_t* tokens, int n_tokens,
                   const dfssm_state* state, void* workspace, void* prefill_workspace, int max_rows,
                   uint16_t* logits, int64_t* next, int fuse_next_embed, void* stream);
 
-/* ---- density-field state (row f4) ------------------------------------------------------- */
+/* ---- density-field state ------------------------------------------------------- */
 /* Quantize SSM state rows at a chunk boundary as training/df_ssm_mamba2_distill_dfw.py:139-165
  * (df_ssd_scan) does after every block_len tokens. The reference applies it in training only.
  * Per row of d_state = 128 fp32 values:

@@ -145,7 +145,7 @@ float or_log1pf(float y) { /* y >= 0 (softplus argument) */
 void or_expf_array(const float* x, float* out, long n) { for (long i = 0; i < n; ++i) out[i] = or_expf(x[i]); }
 void or_log1pf_array(const float* x, float* out, long n) { for (long i = 0; i < n; ++i) out[i] = or_log1pf(x[i]); }
 
-/* ---------------------------------------------------------------- bits (row a2) ------------ */
+/* ---------------------------------------------------------------- bits ------------ */
 
 /* Word j, bit b of row n is column 32j+b; bit 1 -> +1, bit 0 -> -1.
  * export_dfssm.py:34-42 (pack), df_ssm_inference.py:23-29 (unpack), cpu_inference.c:126-128. */
@@ -157,7 +157,7 @@ void or_unpack_bits(const uint32_t* packed, int rows, int kwords, int8_t* out) {
     }
 }
 
-/* ---------------------------------------------------------------- scaffold (row a5) -------- */
+/* ---------------------------------------------------------------- scaffold -------- */
 
 /* byte -> its 8 signs (bit i of the byte -> element i), the unpack of or_unpack_bits 8 at a time */
 static int8_t sign_lut[256][8];
@@ -205,7 +205,7 @@ void or_rmsnorm(const uint16_t* x, const float* w, int M, int K, uint16_t* out) 
   }
 }
 
-/* ---------------------------------------------------------------- quantizer (row a4) ------- */
+/* ---------------------------------------------------------------- quantizer ------- */
 
 /* _quantize_to_int8, df_ssm_inference.py:147-152:
  *   s = fp16(fp16(max(amax|x|, 1e-4)) * (1/127))   (ATen divides a tensor by a CPU scalar
@@ -269,7 +269,7 @@ void or_dequant_lora(const int32_t* acc, const uint16_t* xs, const uint16_t* ws,
     }
 }
 
-/* ---------------------------------------------------------------- conv (row a7) ------------ */
+/* ---------------------------------------------------------------- conv ------------ */
 
 /* conv_step_kernel, df_ssm_kernels.cu:27-47: out = s0*w0 + s1*w1 + s2*w2 + x*w3 + b (fp32,
  * left to right), state <- (s1, s2, x), x <- fp16(out * 1/(1+exp(-out))). Products of two fp16
@@ -295,7 +295,7 @@ void or_conv_step(uint16_t* state, uint16_t* xbc, int ld, const uint16_t* w, con
     }
 }
 
-/* ---------------------------------------------------------------- SSM (row a8) ------------- */
+/* ---------------------------------------------------------------- SSM ------------- */
 
 /* ssm_step_kernel, df_ssm_kernels.cu:53-103, with an fp32 state and P = d_inner/nheads:
  *   dt = log1p(exp(dt_raw + dt_bias)); Abar = exp(dt * -exp(A_log))   (or_expf / or_log1pf)
@@ -333,7 +333,7 @@ void or_ssm_step(float* h, const uint16_t* xbc, int ld_xbc, const uint16_t* dt_r
     }
 }
 
-/* ---------------------------------------------------------------- gate (row a9) ------------ */
+/* ---------------------------------------------------------------- gate ------------ */
 
 /* g = fp16(y * fp16(z * fp16(sigmoid(z)))) -- the three fp16 tensor ops of
  * df_ssm_inference.py:194-195; the gated RMSNorm is or_rmsnorm on g. */
@@ -348,7 +348,7 @@ void or_gate(const uint16_t* y, const uint16_t* z, int ld_z, int M, int DI, uint
     }
 }
 
-/* ---------------------------------------------------------------- residual (row a10) ------- */
+/* ---------------------------------------------------------------- residual ------- */
 
 void or_residual(uint16_t* x, const uint16_t* o, int M, int D) {
   for (long i = 0; i < (long)M * D; ++i) x[i] = or_f2h(hf(x[i]) + hf(o[i]));

@@ -1,4 +1,4 @@
-"""Exporter (row f2): float student weights -> .dfssm, as training/export_dfssm.py converts them.
+"""Exporter: float student weights -> .dfssm, as training/export_dfssm.py converts them.
 
 Pinned by known answers of each conversion (sign bits including exact zeros, mean |w| scale,
 per-row int8 quantization with round-half-even and the 1e-8 floor, LoRA scaling folded into A),

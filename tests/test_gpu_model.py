@@ -1,6 +1,6 @@
 """End-to-end GPU decode parity against the oracle on seeded random-init models.
 
-Per step: fp16 logits identical to the oracle's on the int8 table (the north star allows 2e-2
+Per step: fp16 logits identical to the oracle's on the int8 table (the parity goal allows 2e-2
 absolute), identical greedy tokens; after the run the fp32 SSM state within 1e-3 max relative
 error and the conv state close.
 """

@@ -40,7 +40,7 @@ def _np16(t):
 
 # ------------------------------------------------------------------------------ config 1
 def _lora_op_case(N, K, M, seed):
-    """Inputs of one scaffold + LoRA call (BASELINE config 1 distributions) and its oracle outputs."""
+    """Inputs of one scaffold + LoRA call (the benchmark's distributions) and its oracle outputs."""
     rng = np.random.default_rng([1, N, K, M, seed])
     bits = rng.integers(0, 2**32, (N, K // 32), dtype=np.uint64).astype(np.uint32)
     ws = rng.uniform(0.01, 0.05, N).astype(np.float16)
@@ -75,7 +75,7 @@ def _check_lora_op(out, ref):
 @pytest.mark.parametrize("M", [1, 2, 3, 4, 16, 32])
 @pytest.mark.parametrize("xchg", [True, False])
 def test_scaffold_lora_op_bit_exact(N, K, M, xchg):
-    """packed bits with fp16 row scales ~U(0.01, 0.05), int8 activations
+    """Packed bits with fp16 row scales ~U(0.01, 0.05), int8 activations
     ~N(0, 40) clipped with fp16 per-token scales, rank-16 int8 LoRA A/B; xn is the fp16 vector
     the activations quantize (the LoRA reads it, df_ssm_inference.py:173). xchg: with the exchange
     workspace (one launch at M <= 4), else without."""

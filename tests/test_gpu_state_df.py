@@ -1,4 +1,4 @@
-"""Density-field state (row f4) on the GPU against the oracle (or_state_df).
+"""Density-field state on the GPU against the oracle (or_state_df).
 
 dfssm_state_density_field must reproduce the oracle bit for bit (state and sigma-delta error) on
 random rows of many scales, constant rows and 1.3B-sized state, for power-of-two and other
